@@ -13,7 +13,9 @@
  * what the C++ layer in cuda_matmul.h passes. Calls are queued and return
  * before the GPU finishes. Calls that use split-K share one library-owned
  * scratch buffer: concurrent calls on different streams race, as in the
- * reference (cuda_matmul.h:7-12).
+ * reference (cuda_matmul.h:7-12). (The k slices of automatic's fp32 split
+ * product are the exception: each stream, and each capture, has a buffer of
+ * its own, 2 GiB in all; past that the product runs without slices.)
  *
  * Layout (cuda_matmul.h:94-107): A is m x k, B is k x n, C is m x n, all
  * dense row-major fp32 with no leading dimensions; int8 B carries n fp32
@@ -40,7 +42,9 @@ extern "C" {
 
 /* Kernel choice; replaces enum class GpuKernel, cuda_matmul.h:61-67. */
 #define EM_KERNEL_AUTOMATIC 0   /* fp32 B: skinny for m <= 8 (m <= 3 for 2^25 weights or more),
-                                   else tiled_split (tiled if B is unaligned); int8 B: skinny
+                                   else a six-term bf16 split of both operands on MFMA where it
+                                   is faster (most shapes past 2^20 weights), tiled_split or
+                                   tiled; int8 B: skinny
                                    for 1 row, and for 2-4 rows of small weights, else the
                                    exact-split bf16 MFMA kernel */
 #define EM_KERNEL_NAIVE 1       /* one thread per element of C; the reference kernel */

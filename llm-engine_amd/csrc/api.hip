@@ -8,12 +8,14 @@
 // path can be exercised without a GPU. Errors come back as status codes with
 // a message for em_last_error(); the messages name both shapes as
 // "(A is MxK, B is KxN)", as the reference's exceptions do.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <mutex>
 #include <string>
 #include <type_traits>
 #include <unordered_map>
+#include <vector>
 
 #include "internal.hpp"
 #include "llm_engine_amd.h"
@@ -148,6 +150,7 @@ int matmul_entry(std::size_t m, std::size_t n, std::size_t k, const float* A, co
     // Above that, the B-streaming fp32 MFMA kernel (tiled_split), except
     // where tiled_preferred picks the LDS-tiled GEMM (large m, small B, or
     // wide B from 256 rows): the reference switches to tiled past 64 rows.
+    // Most of those go to the bf16 split kernel instead (gemm_split_preferred).
     // int8 B goes to the exact-split bf16 MFMA
     // kernel instead (split_bf16.hip: at 4096^2, 1.1x faster than
     // tiled_split at m = 9-16 and 1.3-2.6x from m = 32 to 512), and so do
@@ -234,6 +237,11 @@ int matmul_entry(std::size_t m, std::size_t n, std::size_t k, const float* A, co
             a.A = normed;
             a.rms_weight = nullptr;
         }
+        if (!std::is_same<BT, int8_t>::value && automatic && gemm_split_preferred(a)) {
+            run_gemm_split(a);
+            hip_check(hipGetLastError(), "launch");
+            return EM_OK;
+        }
         switch (kernel) {
             case EM_KERNEL_NAIVE: run_naive<BT>(a); break;
             case EM_KERNEL_TILED: run_tiled<BT>(a); break;
@@ -299,6 +307,75 @@ float* scratch(ScratchSlot slot, std::size_t floats) {
         g_generation.fetch_add(1);
     }
     return g_scratch[slot];
+}
+
+namespace {
+
+struct StreamBuffer {
+    int device;
+    hipStream_t stream;
+    unsigned long long thread;   // of a hipStreamPerThread caller, 0 for a stream handle
+    unsigned long long capture;  // capture id, 0 outside one
+    float* p;
+    std::size_t cap;  // floats
+};
+constexpr std::size_t kStreamBuffers = 64, kStreamBytes = std::size_t{2} << 30;
+std::mutex g_stream_mu;
+std::vector<StreamBuffer> g_stream_buffers;
+std::size_t g_stream_bytes = 0;  // kept in all, outgrown buffers included
+
+}  // namespace
+
+float* stream_workspace(hipStream_t stream, std::size_t floats) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    int device = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess ||
+        hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    // A number of its own for each thread, never used again after it ends.
+    static std::atomic<unsigned long long> threads{0};
+    thread_local const unsigned long long number = threads.fetch_add(1) + 1;
+    const unsigned long long me = stream == hipStreamPerThread ? number : 0;
+    if (status == hipStreamCaptureStatusNone) id = 0;
+    std::lock_guard<std::mutex> lock(g_stream_mu);
+    auto it = std::find_if(g_stream_buffers.begin(), g_stream_buffers.end(),
+                           [&](const StreamBuffer& b) {
+                               return b.device == device && b.stream == stream &&
+                                      b.thread == me && b.capture == id;
+                           });
+    if (it != g_stream_buffers.end() && it->cap >= floats) return it->p;
+    // Doubling sizes, so the outgrown buffers add up to less than the last.
+    std::size_t cap = std::size_t{1} << 20;
+    while (cap < floats) cap *= 2;
+    const std::size_t bytes = cap * sizeof(float);
+    if (bytes > kStreamBytes - g_stream_bytes ||
+        (it == g_stream_buffers.end() && g_stream_buffers.size() >= kStreamBuffers))
+        return nullptr;
+    // An allocation is not a stream operation; under a capture it only has
+    // to be allowed.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    void* p = nullptr;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const hipError_t err = hipMalloc(&p, bytes);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_stream_bytes += bytes;
+    if (it == g_stream_buffers.end()) {
+        g_stream_buffers.push_back({device, stream, me, id, static_cast<float*>(p), cap});
+        return static_cast<float*>(p);
+    }
+    it->p = static_cast<float*>(p);
+    it->cap = cap;
+    return it->p;
 }
 
 std::size_t scratch_generation() { return g_generation.load(); }

@@ -34,6 +34,14 @@ enum ScratchSlot { kPartial = 0, kNorm = 1, kQuant = 2, kSplitA = 3, kPartialFro
                    kSlots = 5 };
 float* scratch(ScratchSlot slot, std::size_t floats);
 std::size_t scratch_generation();
+// Device memory of at least `floats` floats that only work queued on
+// `stream` uses (hipStreamPerThread: this thread's; a stream under capture:
+// that capture's), so calls on different streams do not share it, unlike
+// scratch(). Kept for the stream's next call; a buffer that grows is kept
+// too, since a captured graph may hold it. Null, nothing allocated, past 64
+// streams or 2 GiB in all, or if the memory cannot be had: the caller then
+// does without.
+float* stream_workspace(hipStream_t stream, std::size_t floats);
 // Library-owned arrival counters for one-launch split-K products: `count`
 // 32-bit words, zero. Grow-only like scratch() (growth bumps
 // scratch_generation()); zeroed when allocated, and every call leaves the
@@ -125,6 +133,14 @@ void run_tiled(const MatmulArgs& a);
 // 135 / 140; 11008 x 4096 at m = 512 355 / 374, m = 1024 706 / 676;
 // 288 x 768 at m = 9 .. 1024 12-18 / 8.5; 768 x 288 at m = 32 16.2 / 11.8.
 bool tiled_preferred(const MatmulArgs& a);
+
+// fp32 products of more than 8 rows as six bf16 MFMA terms of an exact
+// three-way split of both operands (gemm_split.hip). A must already be
+// normed. supports: k >= 32, k % 4 == 0, A 16-byte aligned. preferred: where
+// automatic takes it over tiled and tiled_split.
+bool gemm_split_supports(const MatmulArgs& a);
+bool gemm_split_preferred(const MatmulArgs& a);
+void run_gemm_split(const MatmulArgs& a);
 
 // One thread per element (GpuKernel::naive). A must already be normed.
 template <class BT>

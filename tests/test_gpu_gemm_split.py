@@ -1,0 +1,124 @@
+"""fp32 products of more than 8 rows through `automatic`, where it splits both
+operands into bf16 terms (csrc/gemm_split.hip), against 64-bit products.
+
+Bound per element: every MFMA adds its 32 products to an fp32 accumulator
+with at most two roundings of 2^-24 each at the size of the sums so far, and
+six terms a chunk in two accumulators of which only hi * hi is full size; the
+slices' sum and the prior C add one each, the left-out terms 2^-26. So
+(k / 16 + 24) * 2^-24 * sum |a||b| holds with room (the sums are rarely at
+their largest throughout)."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from tests import engine, inputs
+
+em = engine.load()
+pytestmark = pytest.mark.gpu
+
+
+def dev(x):
+    return torch.from_numpy(x).cuda()
+
+
+def check(got, A, B, C0=None):
+    k = A.shape[1]
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    scale = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    if C0 is not None:
+        want, scale = want + C0, scale + np.abs(C0)
+    err = np.abs(got.astype(np.float64) - want)
+    assert (err <= (k / 16 + 24) * 2.0 ** -24 * scale + 2.0 ** -149).all(), (err / scale).max()
+
+
+# Rows around every tile height, k whole and ragged chunks (the last one
+# overlapping the one before), columns off a tile, off a float4 and narrow.
+SHAPES = [(9, 1000, 1100), (32, 1028, 1500), (33, 1156, 1000), (64, 4096, 300), (65, 36, 40000),
+          (97, 2000, 700), (128, 1060, 1027), (129, 1000, 1153), (161, 1124, 1000),
+          (193, 1500, 1001), (257, 2048, 1030), (320, 1100, 1000), (321, 1092, 2049),
+          (513, 1028, 2000), (40, 44, 30001), (1100, 32, 40000)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_tile_edges(shape):
+    m, k, n = shape
+    A = inputs.uniform((m, k), -1.0, 1.0, 71)
+    B = inputs.uniform((k, n), -1.0, 1.0, 72)
+    C0 = inputs.uniform((m, n), -4.0, 4.0, 73)
+    first = em.matmul(dev(A), dev(B))
+    check(first.cpu().numpy(), A, B)
+    assert torch.equal(first, em.matmul(dev(A), dev(B)))
+    C = dev(C0.copy())
+    em.matmul(dev(A), dev(B), C, accumulate=True)
+    check(C.cpu().numpy(), A, B, C0)
+    # C off a 16-byte boundary: scalar stores of the same sums.
+    flat = torch.empty(m * n + 1, device="cuda")
+    off = flat[1:].view(m, n)
+    em.matmul(dev(A), dev(B), off)
+    assert torch.equal(off, first)
+
+
+@pytest.mark.parametrize("exponent", [-100, -115, -126, 40])
+def test_magnitudes(exponent):
+    # Below 2^-109 a lo term drops bits; the product must not. With B scaled
+    # the other way the sums stay normal numbers.
+    m, k, n = 70, 1100, 1200
+    A = (inputs.uniform((m, k), 1.0, 2.0, 74) * 2.0 ** exponent).astype(np.float32)
+    A[::2] = inputs.uniform((m, k), -1.0, 1.0, 75)[::2]
+    B = (inputs.uniform((k, n), -1.0, 1.0, 76) * 2.0 ** (20 if exponent < 0 else -100)).astype(np.float32)
+    check(em.matmul(dev(A), dev(B)).cpu().numpy(), A, B)
+    check(em.matmul(dev(np.ascontiguousarray(B.T)), dev(np.ascontiguousarray(A.T))).cpu().numpy(),
+          B.T, A.T)
+
+
+def test_non_finite_values():
+    m, k, n = 130, 1100, 1200
+    A = inputs.uniform((m, k), 0.5, 1.0, 77)
+    B = inputs.uniform((k, n), 0.5, 1.0, 78)
+    A[3, 5], A[70, 1099], B[7, 11], B[1098, 1199] = np.inf, -np.inf, np.inf, np.nan
+    A[5, 9] = np.float32(3.4e38)  # rounds up to infinity as a bf16
+    with np.errstate(invalid="ignore"):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+    got = em.matmul(dev(A), dev(B)).cpu().numpy()
+    over = np.abs(want) > np.finfo(np.float32).max  # past fp32: +inf
+    want[over & np.isfinite(want)] = np.inf
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    fine = np.isfinite(want)
+    assert np.allclose(got[fine], want[fine], rtol=1e-5)
+
+
+def test_streams_and_threads_share_nothing():
+    # Sliced products on four threads with a stream each, and a graph captured
+    # without a call before it: every result equals the first stream's.
+    m, k, n = 200, 4096, 1024
+    A, B = dev(inputs.uniform((m, k), -1, 1, 79)), dev(inputs.uniform((k, n), -1, 1, 80))
+    As = [A * (i + 1) for i in range(4)]
+    want = [em.matmul(a, B).clone() for a in As]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(40):
+                if not torch.equal(em.matmul(As[i], B), want[i]):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
+    out = [torch.zeros((m, n), device="cuda") for _ in range(2)]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        em.matmul(As[0], B, out[0])
+        em.matmul(As[1], B, out[1])
+    for _ in range(3):
+        out[0].zero_(), out[1].zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+        em.matmul(As[2], B)
