@@ -26,7 +26,8 @@
 //    normalised and written by the first kernel; the merge kernel then exits.
 //    With more rows (prefill), automatic runs the tile kernel (16
 //    query rows per wave on fp32 MFMA), split over the context as well when
-//    its grid is small; for head sizes it is not built for, the same split
+//    its grid is small, or for large grids the 64-row kernel (bf16 MFMA, keys
+//    and values shared through LDS); for head sizes it is not built for, the same split
 //    kernel with one chunk per row: the whole context in rounds, no merge.
 //  * single_block (on request): workgroup (head, row) holds the query and
 //    the scores of the whole context in LDS; any head size.
@@ -744,27 +745,18 @@ __device__ __forceinline__ void load_run(const float* src, float* dst) {
 
 constexpr int kTileWaves = 4;
 
+// One wave's online softmax over positions [first, wlast] (both ends of
+// whole 16-position blocks) for the 16 queries r0 + j of head h: max m, this
+// lane's part l of the sum, unnormalised output o. `last` is the last
+// position that may be read.
 template <int E>
-__global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs a) {
+__device__ __forceinline__ void tile_wave(const AttnArgs& a, int h, int r0, int last, int first,
+                                          int wlast, float& m, float& l, floatx4 (&o)[E]) {
     constexpr int HS = 16 * E, Q4 = 4 * E;
     constexpr int KB = 16;  // positions per block
-    __shared__ float ms[kTileWaves][kWave], ls[kTileWaves][kWave];
-    __shared__ floatx4 os[kTileWaves][E][kWave];
     const int lane = threadIdx.x % kWave, g = lane >> 4, j = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // Row tiles in reverse: the longest (causal) start first and the short
-    // ones fill in behind them.
-    const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kTileRows;
-    const int pos0 = *a.pos;
     const int row = min(r0 + j, a.rows - 1);  // rows past the call: computed, not stored
-    const int pq = pos0 + row;                // this lane's query position
-    const int last = pos0 + min(r0 + kTileRows - 1, a.rows - 1);  // the wave's last position
-    // Split over the context: this workgroup takes positions [lo, hi] of
-    // chunk blockIdx.z (none past last: the grid is sized for seq_len).
-    const int cz = blockIdx.z;
-    const int lo = cz * a.tile_chunk;
-    if (lo > last) return;
-    const int hi = a.tile_chunk ? min(last, lo + a.tile_chunk - 1) : last;
+    const int pq = *a.pos + row;              // this lane's query position
     const float* kbase = a.kc + static_cast<std::size_t>((h / a.group) * HS);
     const float* vbase = a.vc + static_cast<std::size_t>((h / a.group) * HS);
 
@@ -787,8 +779,8 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs 
     };
 
     const float scale = 1.0f / sqrtf(static_cast<float>(HS));
-    float m = -INFINITY, l = 0.0f;
-    floatx4 o[E];
+    m = -INFINITY;
+    l = 0.0f;
 #pragma unroll
     for (int c = 0; c < E; ++c) o[c] = floatx4{0.f, 0.f, 0.f, 0.f};
 
@@ -829,11 +821,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs 
         m = mn;
     };
 
-    // This wave's blocks: [nb * w / 4, nb * (w + 1) / 4) of the nb blocks
-    // from lo (a multiple of 16) through hi.
-    const int b0i = lo / KB, nb = hi / KB + 1 - b0i;
-    const int first = KB * (b0i + nb * wave / kTileWaves);
-    const int wlast = KB * (b0i + nb * (wave + 1) / kTileWaves) - 1;  // < first: no blocks
     if (first <= wlast) {
         TileBlock<E> b0, b1;
         load(b0, first);
@@ -845,6 +832,78 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs 
             use(b1, t0 + KB);
         }
     }
+}
+
+// The result of query r0 + j over positions from lo = cz * tile_chunk on:
+// max M, whole sum l, unnormalised output. Split: a query whose context
+// spans more than one chunk leaves this chunk's state for the merge kernel;
+// one whose context fits chunk 0 is written here, as the split kernel writes
+// it. run(u, f) is the float4 of f * the output at head dims run_at(u) ..
+// + 3, u < E.
+template <int E, class At, class Run>
+__device__ __forceinline__ void tile_store(const AttnArgs& a, int h, int r0, int cz, float M,
+                                           float l, At run_at, Run run) {
+    constexpr int HS = 16 * E;
+    const int lane = threadIdx.x % kWave, g = lane >> 4, j = lane & 15;
+    const int pq = *a.pos + min(r0 + j, a.rows - 1), lo = cz * a.tile_chunk;
+    if (r0 + j < a.rows && a.tile_chunk && pq >= a.tile_chunk && lo <= pq) {
+        const std::size_t b = (static_cast<std::size_t>(r0 + j) * a.n_heads + h) * a.splits + cz;
+#pragma unroll
+        for (int u = 0; u < E; ++u)
+            *reinterpret_cast<floatx4*>(a.part_o + b * HS + run_at(u)) = run(u, 1.0f);
+        if (g == 0) a.part_ml[b] = make_float2(M, l);
+    } else if (r0 + j < a.rows && cz == 0 && (a.tile_chunk == 0 || pq < a.tile_chunk)) {
+        const float inv = 1.0f / l;
+        float* dst = a.out + static_cast<std::size_t>(r0 + j) * a.out_stride +
+                     static_cast<std::size_t>(h) * HS;
+#pragma unroll
+        for (int u = 0; u < E; ++u) *reinterpret_cast<floatx4*>(dst + run_at(u)) = run(u, inv);
+    }
+}
+
+// tile_store of tile_wave's layout: o[c][r] is head dim E (4g + r) + c.
+template <int E>
+__device__ __forceinline__ void tile_store_wave(const AttnArgs& a, int h, int r0, int cz, float M,
+                                                float l, const floatx4 (&o)[E]) {
+    float flat[4 * E];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < E; ++c) flat[E * r + c] = o[c][r];
+    const int g = (threadIdx.x % kWave) >> 4;
+    tile_store<E>(a, h, r0, cz, M, l, [&](int u) { return 4 * E * g + 4 * u; },
+                  [&](int u, float f) {
+                      return floatx4{flat[4 * u] * f, flat[4 * u + 1] * f, flat[4 * u + 2] * f,
+                                     flat[4 * u + 3] * f};
+                  });
+}
+
+template <int E>
+__global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs a) {
+    constexpr int KB = 16;  // positions per block
+    __shared__ float ms[kTileWaves][kWave], ls[kTileWaves][kWave];
+    __shared__ floatx4 os[kTileWaves][E][kWave];
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    // Row tiles in reverse: the longest (causal) start first and the short
+    // ones fill in behind them.
+    const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kTileRows;
+    const int last = *a.pos + min(r0 + kTileRows - 1, a.rows - 1);  // the tile's last position
+    // Split over the context: this workgroup takes positions [lo, hi] of
+    // chunk blockIdx.z (none past last: the grid is sized for seq_len).
+    const int cz = blockIdx.z;
+    const int lo = cz * a.tile_chunk;
+    if (lo > last) return;
+    const int hi = a.tile_chunk ? min(last, lo + a.tile_chunk - 1) : last;
+
+    // This wave's blocks: [nb * w / 4, nb * (w + 1) / 4) of the nb blocks
+    // from lo (a multiple of 16) through hi.
+    const int b0i = lo / KB, nb = hi / KB + 1 - b0i;
+    const int first = KB * (b0i + nb * wave / kTileWaves);
+    const int wlast = KB * (b0i + nb * (wave + 1) / kTileWaves) - 1;  // < first: no blocks
+    float m, l;
+    floatx4 o[E];
+    tile_wave<E>(a, h, r0, last, first, wlast, m, l, o);
 
     // Merge the waves in order: lane l of every wave holds query j's state.
     ms[wave][lane] = m;
@@ -874,34 +933,315 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs 
     // the xor pairs add them in the same order in every lane.
     l += __shfl_xor(l, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
-    // Split: a query whose context spans more than one chunk leaves this
-    // chunk's (max, sum, unnormalised output) for the merge kernel; one whose
-    // context fits chunk 0 is written here, as the split kernel writes it.
-    if (r0 + j < a.rows && a.tile_chunk && pq >= a.tile_chunk && lo <= pq) {
-        const std::size_t b = (static_cast<std::size_t>(r0 + j) * a.n_heads + h) * a.splits + cz;
-        floatx4* dst = reinterpret_cast<floatx4*>(a.part_o + b * HS + Q4 * g);
-        float run[Q4];
+    tile_store_wave<E>(a, h, r0, cz, M, l, o);
+}
+
+// --- prefill rows: tiles of 64 queries on bf16 MFMA -------------------------
+//
+// Workgroup (query head, 64 rows): wave w has the 16 queries r0 + 16w + j.
+// The tile kernel above reads every key and value once per 16 rows (1 GB of
+// L2 reads for 1000 rows of 32 heads) and multiplies on fp32 MFMA at 32
+// cycles per 16x16x4; here the four waves share each 32-position block
+// through LDS, and both products are sums of six bf16 terms: every operand
+// (Q, K, V and the softmax weights P) split exactly into three bf16 values,
+// the terms above 2^-26 of a product kept, hi * hi in an accumulator of its
+// own (gemm_split.hip has the error argument; here 1.5e-7 off
+// 64 bits against 1.9e-7). 1000 rows x 32 heads of 128
+// at context 1000: 85 us against 140.
+//
+// A block's keys and values are loaded into registers one block ahead,
+// split, and written to LDS between two barriers; two workgroups share a CU,
+// so one's split and softmax run beside the other's MFMAs. In lane
+// (g, j) of a wave:
+//  * S^T = K Q^T (positions x queries): the keys are the first operand, in
+//    16-position fragments of 32 head dims with the 16-byte units of a row
+//    permuted by unit ^ (row / 2 % 4); Q's terms stay in registers. Head
+//    dims past the head size (16, 48, 80, 112) are zeros.
+//  * The lane ends with query j's scores at positions 4g + r of both halves
+//    of the block, r < 4. They are its eight k values for O^T += V^T P^T
+//    once V's fragments take the positions in that order (slot 8g + e is
+//    position 4g + e, or 16 + 4g + e - 4 from e = 4), so scores never leave
+//    the lane.
+//  * O^T block c: head dims 16c + 4g + r of query j.
+// The output is rescaled only when a maximum of the wave's queries moved.
+//
+// Terms below 2^-133 drop bits: scores are never that sensitive, but a value
+// (or a weight) that small may be all of an output. Where bits of V were
+// dropped and an output's sum is below 2^-50 (of P, and it is also not
+// zero), or an output or sum is not finite, the wave runs tile_wave instead.
+constexpr int kRowsTile = 64;
+constexpr int kRowsBlock = 32;
+
+// e^x for x <= 0 (NaN stays, 0 below 2^-126): 2^(x log2 e) with the
+// rounding of the product and the rest of log2 e put back as a factor, within
+// about 2 ulp in half of expf's instructions.
+__device__ __forceinline__ float exp_neg(float x) {
+    constexpr float kHi = 0x1.715476p+0f, kLo = 0x1.4ae0cp-26f, kLn2 = 0x1.62e43p-1f;
+    const float t = x < -200.0f ? -200.0f : x;
+    const float y = t * kHi;
+    const float r = fmaf(t, kLo, fmaf(t, kHi, -y));
+    const float p = __builtin_amdgcn_exp2f(y);
+    return fmaf(p, r * kLn2, p);
+}
+
+template <int E>
+__global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
+    constexpr int HS = 16 * E, C = (HS + 31) / 32, T = 4 * kWave;
+    constexpr int kKeys = C * 2 * 3 * 1024, kTerm = HS * 64;  // bytes; a term of V
+    __shared__ __attribute__((aligned(1024))) char smem[kKeys + 3 * kTerm];
+    const int tid = threadIdx.x, lane = tid % kWave, g = lane >> 4, j = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    // Longest (causal) tiles first.
+    const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kRowsTile;
+    const int pos0 = *a.pos;
+    const int last = pos0 + min(r0 + kRowsTile - 1, a.rows - 1);
+    const int wr0 = r0 + 16 * w;
+    const int row = min(wr0 + j, a.rows - 1);  // rows past the call: computed, not stored
+    const int pq = pos0 + row;                 // the lane's query position
+    const int wlast = pos0 + min(wr0 + 15, a.rows - 1);  // the wave's last one
+    const float* kbase = a.kc + static_cast<std::size_t>((h / a.group) * HS);
+    const float* vbase = a.vc + static_cast<std::size_t>((h / a.group) * HS);
+
+    uint32_t lost_q = 0, lost_v = 0, lost_p = 0;  // lost_q is not used: see above
+    bf16x8 q[C][3];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < C; ++c) {
+        const float* src = a.q + static_cast<std::size_t>(row) * a.q_stride +
+                           static_cast<std::size_t>(h) * HS + min(32 * c + 8 * g, HS - 8);
+        const floatx4 x0 = *reinterpret_cast<const floatx4*>(src);
+        const floatx4 x1 = *reinterpret_cast<const floatx4*>(src + 4);
+        const bool in = 32 * c + 8 * g < HS;
+        float v[8];
 #pragma unroll
-            for (int c = 0; c < E; ++c) run[E * r + c] = o[c][r];
+        for (int e = 0; e < 4; ++e) {
+            v[e] = in ? x0[e] : 0.0f;
+            v[4 + e] = in ? x1[e] : 0.0f;
+        }
+        uint4 t[3];
+        split3x8(v, t, lost_q);
 #pragma unroll
-        for (int u = 0; u < E; ++u)
-            dst[u] = floatx4{run[4 * u], run[4 * u + 1], run[4 * u + 2], run[4 * u + 3]};
-        if (g == 0) a.part_ml[b] = make_float2(M, l);
-    } else if (r0 + j < a.rows && cz == 0 && (a.tile_chunk == 0 || pq < a.tile_chunk)) {
-        const float inv = 1.0f / l;
-        floatx4* dst = reinterpret_cast<floatx4*>(a.out + static_cast<std::size_t>(r0 + j) * a.out_stride +
-                                                  static_cast<std::size_t>(h) * HS + Q4 * g);
-        float run[Q4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < E; ++c) run[E * r + c] = o[c][r] * inv;
-#pragma unroll
-        for (int u = 0; u < E; ++u)
-            dst[u] = floatx4{run[4 * u], run[4 * u + 1], run[4 * u + 2], run[4 * u + 3]};
+        for (int x = 0; x < 3; ++x) q[c][x] = __builtin_bit_cast(bf16x8, t[x]);
     }
+
+    // The block at t0 covers positions t0 .. t0 + 31; one that would pass
+    // `last` starts at last - 31 instead (>= 0: the call has 32 rows or
+    // more), its positions before t0 masked, so no load needs a bound.
+    auto start = [&](int t0) { return min(t0, last - (kRowsBlock - 1)); };
+    // Keys: wave-task x = w, w + 4, ... is (head dims 32 (x / 2), positions
+    // 16 (x % 2)): lane l loads unit l % 4 of position l / 4.
+    constexpr int NK = (2 * C + 3) / 4;
+    const int jr = lane / 4, uu = lane % 4;
+    int k_off[NK];
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+        const int x = min(w + 4 * i, 2 * C - 1);
+        k_off[i] = (16 * (x % 2) + jr) * a.kv_stride + min(32 * (x / 2) + 8 * uu, HS - 8);
+    }
+    // Values: task t is (slot group t / HS, head dim t % HS).
+    constexpr int NV = (4 * HS + T - 1) / T;
+    int v_off[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int t = min(tid + i * T, 4 * HS - 1);
+        v_off[i] = 4 * (t / HS) * a.kv_stride + t % HS;
+    }
+    floatx4 kr[NK][2];
+    float vr[NV][8];
+    auto load = [&](int t0) {
+        const float* kp = kbase + static_cast<std::size_t>(start(t0)) * a.kv_stride;
+        const float* vp = vbase + static_cast<std::size_t>(start(t0)) * a.kv_stride;
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            kr[i][0] = *reinterpret_cast<const floatx4*>(kp + k_off[i]);
+            kr[i][1] = *reinterpret_cast<const floatx4*>(kp + k_off[i] + 4);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                vr[i][e] = vp[static_cast<std::size_t>(e < 4 ? e : 12 + e) * a.kv_stride + v_off[i]];
+    };
+    auto stash = [&] {
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int x = w + 4 * i;
+            if ((2 * C) % 4 && x >= 2 * C) break;
+            float v[8] = {kr[i][0].x, kr[i][0].y, kr[i][0].z, kr[i][0].w,
+                          kr[i][1].x, kr[i][1].y, kr[i][1].z, kr[i][1].w};
+            if (HS % 32 && x / 2 == C - 1) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = 32 * (C - 1) + 8 * uu < HS ? v[e] : 0.0f;
+            }
+            uint4 t[3];
+            split3x8(v, t, lost_q);
+            char* o = smem + x * 3072 + (jr * 4 + (uu ^ ((jr >> 1) & 3))) * 16;
+#pragma unroll
+            for (int y = 0; y < 3; ++y) *reinterpret_cast<uint4*>(o + y * 1024) = t[y];
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int x = tid + i * T;
+            if ((4 * HS) % T && x >= 4 * HS) break;
+            uint4 t[3];
+            split3x8(vr[i], t, lost_v);
+#pragma unroll
+            for (int y = 0; y < 3; ++y)
+                *reinterpret_cast<uint4*>(smem + kKeys + y * kTerm + x * 16) = t[y];
+        }
+    };
+
+    const float scale = 1.0f / sqrtf(static_cast<float>(HS));
+    float m = -INFINITY, l = 0.0f;
+    floatx4 o[E], ol[E];  // the V hi * P hi products; the five smaller ones
+#pragma unroll
+    for (int c = 0; c < E; ++c) o[c] = ol[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const char* k_rd = smem + (j * 4 + (g ^ ((j >> 1) & 3))) * 16;
+    const char* v_rd = smem + kKeys + (g * HS + j) * 16;
+
+    auto use = [&](int t0) {
+        // Scores of the block's two halves.
+        floatx4 sh[2][2], sl[2];  // hi * hi in two accumulators, of even and odd dims' chunks
+#pragma unroll
+        for (int p = 0; p < 2; ++p) sh[0][p] = sh[1][p] = sl[p] = floatx4{0.f, 0.f, 0.f, 0.f};
+        bf16x8 k[2][2][3], v[4][3];  // this step's fragments and the next's
+        auto read_k = [&](int c) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int y = 0; y < 3; ++y)
+                    k[c & 1][p][y] =
+                        *reinterpret_cast<const bf16x8*>(k_rd + ((2 * c + p) * 3 + y) * 1024);
+        };
+        auto read_v = [&](int c0) {
+#pragma unroll
+            for (int c = c0; c < c0 + 2 && c < E; ++c)
+#pragma unroll
+                for (int y = 0; y < 3; ++y)
+                    v[c & 3][y] = *reinterpret_cast<const bf16x8*>(v_rd + y * kTerm + c * 256);
+        };
+        read_k(0);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            if (c + 1 < C) read_k(c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            auto mma = [&](floatx4 (&d)[2], int tk, int tq) {
+#pragma unroll
+                for (int p = 0; p < 2; ++p) d[p] = mfma16x16x32(k[c & 1][p][tk], q[c][tq], d[p]);
+            };
+            mma(sh[c & 1], 0, 0);
+            mma(sl, 2, 0);
+            mma(sl, 1, 0);
+            mma(sl, 0, 1);
+            mma(sl, 1, 1);
+            mma(sl, 0, 2);
+        }
+        read_v(0);
+        float s[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) 
+            s[e] = (sh[0][e / 4][e % 4] + sh[1][e / 4][e % 4] + sl[e / 4][e % 4]) * scale;
+        const int ts = start(t0);
+        if (ts != t0 || t0 + kRowsBlock - 1 > pos0 + wr0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int t = ts + 4 * g + (e < 4 ? e : 12 + e);
+                s[e] = t >= t0 && t <= pq ? s[e] : -INFINITY;
+            }
+        }
+        float mb = s[0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) mb = fmaxf(mb, s[e]);
+        mb = max32(max16(mb));
+        // mn = -inf: no position of this query yet; everything stays.
+        const float mn = fmaxf(m, mb);
+        if (__ballot(mn > m)) {
+            const float alpha = mn == -INFINITY ? 1.0f : expf(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int c = 0; c < E; ++c) {
+                o[c] *= alpha;
+                ol[c] *= alpha;
+            }
+            m = mn;
+        }
+        const float base = mn == -INFINITY ? 0.0f : mn;
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            p[e] = exp_neg(s[e] - base);
+            l += p[e];
+        }
+        uint4 t[3];
+        split3x8(p, t, lost_p);
+        bf16x8 pt[3];
+#pragma unroll
+        for (int y = 0; y < 3; ++y) pt[y] = __builtin_bit_cast(bf16x8, t[y]);
+        // Two output blocks at a time, so that an MFMA does not wait for the
+        // one before it.
+#pragma unroll
+        for (int c = 0; c < E; c += 2) {
+            if (c + 2 < E) read_v(c + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            auto mma = [&](floatx4 (&d)[E], int tv, int tp) {
+#pragma unroll
+                for (int y = c; y < c + 2 && y < E; ++y) d[y] = mfma16x16x32(v[y & 3][tv], pt[tp], d[y]);
+            };
+            mma(o, 0, 0);
+            mma(ol, 2, 0);
+            mma(ol, 1, 0);
+            mma(ol, 0, 1);
+            mma(ol, 1, 1);
+            mma(ol, 0, 2);
+        }
+    };
+
+    load(0);
+    for (int t0 = 0; t0 <= last; t0 += kRowsBlock) {
+        __syncthreads();  // the previous block has been read
+        stash();
+        if (t0 + kRowsBlock <= last) load(t0 + kRowsBlock);
+        __syncthreads();
+        if (t0 <= wlast) use(t0);
+    }
+
+    // The four lane groups of query j hold parts of its sum.
+    l = sum32(sum16(l));
+    bool bad = !(l < INFINITY), tiny = false, small = false;
+#pragma unroll
+    for (int c = 0; c < E; ++c) {
+        o[c] += ol[c];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = fabsf(o[c][e]);
+            bad |= !(x < INFINITY);
+            tiny |= x < 0x1p-50f;
+            small |= x < 0x1p-50f && x > 0.0f;
+        }
+    }
+    const bool v_lost = __syncthreads_or((lost_v & 0xffffu) != 0) != 0;
+    const bool p_lost = __ballot((lost_p & 0xffffu) != 0) != 0;
+    if (__ballot(bad || (v_lost && tiny) || (p_lost && small))) {
+        tile_wave<E>(a, h, wr0, wlast, 0, wlast / 16 * 16 + 15, m, l, o);
+        l = sum32(sum16(l));
+        tile_store_wave<E>(a, h, wr0, 0, m, l, o);
+        return;
+    }
+    tile_store<E>(a, h, wr0, 0, m, l, [&](int u) { return 16 * u + 4 * g; },
+                  [&](int u, float f) { return o[u] * f; });
+}
+
+// Where the 64-row kernel takes a tile-kernel call: one workgroup per CU and
+// more without chunks of the context, as the position is not known here and a
+// prompt's context may be no longer than its rows. 32 heads of 128, old / this
+// kernel, us: 512 rows at context 512 / 1024 / 4096 46 / 42, 94 / 77, 380 /
+// 301; 1024 rows 137 / 86 and at 4096 706 / 371; 256 rows at 1024 56 / 80.
+// Heads of 64 (half the MFMAs beside the same softmax): 1024 rows at 1024 /
+// 4096 54 / 49, 329 / 224, but 512 rows 47 / 54; of 48, 1024 rows of 6 heads
+// 31 / 50.
+bool rows_preferred(const AttnShape& s, int rows) {
+    const long long tiles = static_cast<long long>(s.n_heads) * ((rows + kRowsTile - 1) / kRowsTile);
+    return rows >= kRowsBlock &&
+           (s.head_size >= 112 ? tiles >= cu_count() : s.head_size >= 64 && tiles >= 2 * cu_count());
 }
 
 void launch_tile(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t stream) {
@@ -1041,6 +1381,17 @@ void run_attention(const AttnShape& s, int rows, const int* pos, const float* q,
                    const float* vc, float* out, float* scratch, int kernel, hipStream_t stream) {
     kernel = resolve(kernel, rows, s);
     AttnArgs a = base_args(s, rows, pos, q, kc, vc, out);
+    if (kernel == kAttnTile && rows_preferred(s, rows)) {
+        const dim3 grid(s.n_heads, (rows + kRowsTile - 1) / kRowsTile), block(4 * kWave);
+        switch (s.head_size / 16) {
+            case 4: hipLaunchKernelGGL(attn_rows_kernel<4>, grid, block, 0, stream, a); break;
+            case 5: hipLaunchKernelGGL(attn_rows_kernel<5>, grid, block, 0, stream, a); break;
+            case 6: hipLaunchKernelGGL(attn_rows_kernel<6>, grid, block, 0, stream, a); break;
+            case 7: hipLaunchKernelGGL(attn_rows_kernel<7>, grid, block, 0, stream, a); break;
+            default: hipLaunchKernelGGL(attn_rows_kernel<8>, grid, block, 0, stream, a); break;
+        }
+        return;
+    }
     if (kernel == kAttnTile) {
         // The context split needs the caller's scratch (sized by
         // attention_scratch_floats); without it the grid stays whole.

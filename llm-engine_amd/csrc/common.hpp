@@ -88,6 +88,20 @@ __device__ __forceinline__ float fold16(float x, float y) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Sum and maximum of x over lanes l and l ^ 32 (l ^ 16), in both.
+__device__ __forceinline__ float sum32(float x) { return fold32(x, x); }
+__device__ __forceinline__ float sum16(float x) { return fold16(x, x); }
+__device__ __forceinline__ float max32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                    false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float max16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                    false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // DPP move inside rows of 16 lanes: row_shl:8 (0x108) reads lane + 8,
 // row_shr:8 (0x118) lane - 8, row_shl:4 (0x104) lane + 4, row_shr:4 (0x114)
 // lane - 4. The control must be a constant of the instruction.
@@ -369,6 +383,44 @@ __device__ __forceinline__ TileId tile_of(int id, int total, int row_tiles, int 
     t.slice = (idx / col_tiles) % (total / (row_tiles * col_tiles));
     t.row = idx / (total / row_tiles);
     return t;
+}
+
+__device__ __forceinline__ uint32_t bits(float f) { return __builtin_bit_cast(uint32_t, f); }
+__device__ __forceinline__ float from_bits(uint32_t u) { return __builtin_bit_cast(float, u); }
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// (a, b) rounded to nearest bf16, a in the low half.
+__device__ __forceinline__ uint32_t to_bf16x2(float a, float b) {
+    uint32_t r;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Eight fp32 values as three terms of eight bf16, each term the remainder
+// so far rounded to nearest: v = t[0] + t[1] + t[2] exactly for |v| >=
+// 2^-109. `lost` gets bits in its low half when a last term is not the
+// whole remainder (smaller values).
+__device__ __forceinline__ void split3x8(const float (&v)[8], uint4 (&t)[3], uint32_t& lost) {
+#pragma clang fp contract(off)
+    uint32_t h[4], md[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float a = v[2 * e], b = v[2 * e + 1];
+        h[e] = to_bf16x2(a, b);
+        const float ra = a - from_bits(h[e] << 16), rb = b - from_bits(h[e] & 0xffff0000u);
+        md[e] = to_bf16x2(ra, rb);
+        const float sa = ra - from_bits(md[e] << 16), sb = rb - from_bits(md[e] & 0xffff0000u);
+        lost |= bits(sa) | bits(sb);
+        l[e] = to_bf16x2(sa, sb);
+    }
+    t[0] = make_uint4(h[0], h[1], h[2], h[3]);
+    t[1] = make_uint4(md[0], md[1], md[2], md[3]);
+    t[2] = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+__device__ __forceinline__ floatx4 mfma16x16x32(bf16x8 a, bf16x8 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
 __device__ __forceinline__ floatx4 mfma16x16x4(float a, float b, floatx4 c) {

@@ -51,8 +51,6 @@
 namespace em {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
 constexpr int kChunk = 32;  // k rows per step
 
 struct GsParams {
@@ -63,36 +61,6 @@ struct GsParams {
     int direct, accumulate, vec;  // vec: float4 access to out
     int row_tiles, col_tiles;
 };
-
-__device__ __forceinline__ uint32_t bits(float f) { return __builtin_bit_cast(uint32_t, f); }
-__device__ __forceinline__ float from_bits(uint32_t u) { return __builtin_bit_cast(float, u); }
-
-// (a, b) rounded to nearest bf16, a in the low half.
-__device__ __forceinline__ uint32_t to_bf16x2(float a, float b) {
-    uint32_t r;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
-// Eight fp32 values as three terms of eight bf16. `lost` gets bits in its
-// low half when a lo term is not the whole remainder.
-__device__ __forceinline__ void split8(const float (&v)[8], uint4 (&t)[3], uint32_t& lost) {
-#pragma clang fp contract(off)
-    uint32_t h[4], md[4], l[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float a = v[2 * e], b = v[2 * e + 1];
-        h[e] = to_bf16x2(a, b);
-        const float ra = a - from_bits(h[e] << 16), rb = b - from_bits(h[e] & 0xffff0000u);
-        md[e] = to_bf16x2(ra, rb);
-        const float sa = ra - from_bits(md[e] << 16), sb = rb - from_bits(md[e] & 0xffff0000u);
-        lost |= bits(sa) | bits(sb);
-        l[e] = to_bf16x2(sa, sb);
-    }
-    t[0] = make_uint4(h[0], h[1], h[2], h[3]);
-    t[1] = make_uint4(md[0], md[1], md[2], md[3]);
-    t[2] = make_uint4(l[0], l[1], l[2], l[3]);
-}
 
 // The wave's MB x NB blocks of 16 x 16 outputs over k in [kb, ke) by fp32
 // MFMAs on operands from global memory, through put(mb, nb, sums) as the
@@ -177,7 +145,7 @@ __global__ __launch_bounds__(kWave * WR * WC, 2) void gemm_split_kernel(GsParams
                 for (int e = 0; e < 8; ++e) v[e] = (t % 4) * 8 + e < z ? 0.0f : v[e];
             }
             uint4 x[3];
-            split8(v, x, lost);
+            split3x8(v, x, lost);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(o + q * 1024) = x[q];
         }
@@ -206,7 +174,7 @@ __global__ __launch_bounds__(kWave * WR * WC, 2) void gemm_split_kernel(GsParams
         for (int i = 0; i < NT; ++i) {
             if (kTasksB % T && w + i * (T / kWave) >= kTasksB / kWave) break;
             uint4 x[3];
-            split8(rb[i], x, lost);
+            split3x8(rb[i], x, lost);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
                 *reinterpret_cast<uint4*>(smem + 2 * kAStage + s * kBStage + q * (BN * 64) +
@@ -245,8 +213,7 @@ __global__ __launch_bounds__(kWave * WR * WC, 2) void gemm_split_kernel(GsParams
             auto mma = [&](floatx4 (&d)[MB], int tb, int ta) {
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
-                    d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[nb & 1][tb], a[mb][ta],
-                                                                    d[mb], 0, 0, 0);
+                    d[mb] = mfma16x16x32(b[nb & 1][tb], a[mb][ta], d[mb]);
             };
             mma(acc[nb], 0, 0);
             mma(low[nb], 2, 0);

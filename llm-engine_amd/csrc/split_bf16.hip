@@ -65,7 +65,6 @@
 namespace em {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kTile = 256;               // columns per workgroup
 constexpr int kChunk = 32;               // k rows per MFMA step of a wave
@@ -80,8 +79,6 @@ __device__ __forceinline__ int granule(int q) { return q ^ ((q >> 3) & 7); }
 
 // --- A -> three bf16 planes -------------------------------------------------
 
-__device__ __forceinline__ uint32_t bits(float f) { return __builtin_bit_cast(uint32_t, f); }
-__device__ __forceinline__ float from_bits(uint32_t u) { return __builtin_bit_cast(float, u); }
 
 // a = hi + mid + lo exactly for |a| >= 2^-110; each part's bits are the top
 // half of an fp32. +-inf: hi = a, mid = lo = 0 (a - hi would be NaN).

@@ -53,7 +53,6 @@
 namespace em {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kCols = 64;        // columns per workgroup: four strips
 constexpr int kStripCols = 16;
@@ -80,8 +79,6 @@ struct SsParams {
     unsigned* count;    // [tile] arrival counters, zero between calls
 };
 
-__device__ __forceinline__ uint32_t bits(float f) { return __builtin_bit_cast(uint32_t, f); }
-__device__ __forceinline__ float from_bits(uint32_t u) { return __builtin_bit_cast(float, u); }
 
 // Eight fp32 values -> three bf16 terms, packed as MFMA A operands (the
 // arithmetic of split_bf16.hip's split8): hi = the value's top half, mid =
