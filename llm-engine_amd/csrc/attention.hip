@@ -190,6 +190,7 @@ int resolve(int kernel, std::size_t rows, const AttnShape& s) {
 struct AttnArgs {
     int n_heads, head_size, group, seq_len, splits, chunk_cap, rows;
     int min_chunk;   // split_chunk's least chunk for this shape
+    int whole;       // contexts of up to this many positions are one chunk
     int merge_from;  // the merge kernel takes rows of at least this many chunks (>= 2)
     int tile_chunk;  // tile kernel split over the context: positions per chunk (0: no split)
     int q_stride, kv_stride, out_stride;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
     const int hs = a.head_size, hs4 = hs / 4;
     const int hg = blockIdx.x, i = blockIdx.y, s = blockIdx.z;
     const int n_ctx = *a.pos + i + 1;
-    const int chunk = split_chunk(n_ctx, a.splits, a.min_chunk);
+    const int chunk = n_ctx <= a.whole ? n_ctx : split_chunk(n_ctx, a.splits, a.min_chunk);
     const int t0 = s * chunk;
     if (t0 >= n_ctx) return;  // uniform across the workgroup
     const int len = min(chunk, n_ctx - t0);
@@ -571,7 +572,9 @@ __global__ __launch_bounds__(kThreads) void attn_merge_kernel(AttnArgs a) {
     const int h = blockIdx.x / groups, d0 = (blockIdx.x % groups) * dpw;
     const int i = blockIdx.y;
     const int n_ctx = *a.pos + i + 1;
-    const int chunk = a.tile_chunk ? a.tile_chunk : split_chunk(n_ctx, a.splits, a.min_chunk);
+    const int chunk = a.tile_chunk       ? a.tile_chunk
+                      : n_ctx <= a.whole ? n_ctx
+                                         : split_chunk(n_ctx, a.splits, a.min_chunk);
     const int n = (n_ctx + chunk - 1) / chunk;
     if (n < a.merge_from) return;  // one chunk: written by the split kernel; few: by their consumer
     const std::size_t b = (static_cast<std::size_t>(i) * a.n_heads + h) * a.splits;
@@ -1431,7 +1434,7 @@ void run_attention(const AttnShape& s, int rows, const int* pos, const float* q,
 bool run_attention_rope(const AttnShape& s, const int* pos, const Summed& src, int dim,
                         int kv_dim, const float* cos_t, const float* sin_t, float* kc, float* vc,
                         float* out, float* scratch, hipStream_t stream, SplitRow* defer,
-                        bool merge_inside) {
+                        bool merge_inside, int whole) {
     if (resolve(kAttnAutomatic, 1, s) != kAttnSplit || split_lds(s, true, true) > kMaxLds)
         return false;
     if (src.n % 4 || src.mn % 4 || dim % 4 || kv_dim % 4) return false;
@@ -1439,6 +1442,7 @@ bool run_attention_rope(const AttnShape& s, const int* pos, const Summed& src, i
         return false;
     AttnArgs a = base_args(s, 1, pos, nullptr, kc, vc, out);
     set_split(s, 1, scratch, a);
+    if (!defer) a.whole = whole;
     a.src = src;
     a.dim = dim;
     a.kv_dim = kv_dim;
@@ -1466,6 +1470,10 @@ bool run_attention_rope(const AttnShape& s, const int* pos, const Summed& src, i
 }
 
 bool attention_merge_inside_preferred(const AttnShape& s) { return heads_per_block(s) == 1; }
+
+int attention_whole_context(const AttnShape& s) {
+    return heads_per_block(s) == 1 && s.head_size <= 64 ? 256 : 0;
+}
 
 void run_attention_merge(const AttnShape& s, const SplitRow& r, float* out, hipStream_t stream) {
     AttnArgs a = base_args(s, 1, r.pos, nullptr, nullptr, nullptr, out);

@@ -284,7 +284,14 @@ void run_attention(const AttnShape& s, int rows, const int* pos, const float* q,
 bool run_attention_rope(const AttnShape& s, const int* pos, const Summed& src, int dim,
                         int kv_dim, const float* cos_t, const float* sin_t, float* kc, float* vc,
                         float* out, float* scratch, hipStream_t stream,
-                        SplitRow* defer = nullptr, bool merge_inside = false);
+                        SplitRow* defer = nullptr, bool merge_inside = false, int whole = 0);
+// The `whole` to pass for a strip decode step (no defer): contexts of up to
+// this many positions stay in one workgroup per head, whose rounds cost less
+// than the merge of two to four chunks while a head's keys are short.
+// stories15M (6 heads of 48), int8, us per token at context 100 / 120 / 200
+// 149 / 155 / 155 -> 145 / 145 / 150; 16 heads of 64 at 120 / 200 117 / 118
+// -> 108 / 114; heads of 128 at 200 88 -> 90, so those keep their chunks.
+int attention_whole_context(const AttnShape& s);
 // True where the split attention launch should merge a row's chunks itself
 // (merge_inside) rather than leave them to the merge kernel: where one
 // workgroup serves one head. With a group of heads per workgroup the last

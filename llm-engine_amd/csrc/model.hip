@@ -914,7 +914,7 @@ void Model::enqueue(int n) {
                              static_cast<std::size_t>(qkv_cols)};
             if (!run_attention_rope(shape_, feed_dev_.p, qkv, D, KV, rope_cos_.p, rope_sin_.p,
                                     L.kcache.p, L.vcache.p, att_.p, attn_scratch_.p, stream_,
-                                    nullptr, merge_inside_)) {
+                                    nullptr, merge_inside_, attention_whole_context(shape_))) {
                 hipLaunchKernelGGL(rope_cache_kernel, dim3(ceil_div(rope_threads, kThreads), 1),
                                    dim3(kThreads), 0, stream_, qkv, qkv_cols, D, KV, hs,
                                    feed_dev_.p, rope_cos_.p, rope_sin_.p, qkv_.p, L.kcache.p,
