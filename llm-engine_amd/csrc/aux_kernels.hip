@@ -9,7 +9,8 @@
 //                   captured graph holds no memset node
 //   quantize_q8     quant.cpp:6-28 on the GPU, bit-exact: column absmax in
 //                   slices + an order-free max, then scale = absmax / 127 and
-//                   inv = 1 / scale with IEEE division, then
+//                   inv = 1 / scale with IEEE division (in a launch of their
+//                   own for large matrices), then
 //                   q = clamp(round-half-away(B * inv), -127, 127)
 //   dequantize_q8   quant.cpp:30-36
 //   stream_read     a read-only pass over a buffer (probes.hip's read kernel
@@ -92,104 +93,170 @@ __global__ __launch_bounds__(kThreads) void fill_zero_kernel(float* p, size_t co
 
 // --- quantize_q8 -----------------------------------------------------------
 
-// Column maxima of |B| over one slice of rows: partial[slice][c]. With V4
-// (cols % 4 == 0, B 16-byte aligned) a thread owns four adjacent columns
-// and reads them as one float4; eight rows are loaded before any is used.
-template <bool V4>
-__global__ __launch_bounds__(kThreads) void colmax_kernel(int rows, int cols, int span,
+// A thread of both kernels owns four adjacent columns, 4 idx .. + 3, and reads
+// them as one 16-byte load (4-byte aligned: a row of any width starts on a
+// float), all rows of a round in flight before any is used. The last group
+// of a width that is not whole groups is shifted back to end at the last
+// column: its columns are then also another thread's, with the same result.
+struct __attribute__((packed, aligned(4))) Floats4 {
+    float v[4];
+};
+
+__device__ __forceinline__ int column_group(int idx, int cols) { return min(4 * idx, cols - 4); }
+
+constexpr int kQuantRound = 16;  // rows in flight per thread
+
+// Column maxima of |B| over one slice of rows: partial[slice][4 idx + e] of
+// column column_group(idx) + e, `stride` floats to a slice. Bound by the read
+// of B (4096 x 11008: 180 MB).
+__global__ __launch_bounds__(kThreads) void colmax_kernel(int rows, int cols, int span, int stride,
                                                           const float* B, float* partial) {
-    constexpr int W = V4 ? 4 : 1;
-    const int c = (blockIdx.x * kThreads + threadIdx.x) * W;
-    if (c >= cols) return;
+    const int idx = blockIdx.x * kThreads + threadIdx.x;
+    if (4 * idx >= stride) return;
+    const float* col = B + column_group(idx, cols);
     const int r0 = blockIdx.y * span, r1 = min(rows, r0 + span);
     // fmaxf keeps the running value when |B| is NaN, as std::max(scale, v)
-    // does in quant.cpp:14; on ordered values max is exact in any order.
-    float mx[W];
+    // does in quant.cpp:14; on ordered values max is exact in any order, so
+    // the last round may read its last row again.
+    float mx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r = r0; r < r1; r += kQuantRound) {
+        Floats4 x[kQuantRound];
 #pragma unroll
-    for (int e = 0; e < W; ++e) mx[e] = 0.0f;
-    auto take = [&](int r) {
-        const float* row = B + static_cast<size_t>(r) * cols + c;
-        if constexpr (V4) {
-            const float4 v = *reinterpret_cast<const float4*>(row);
-            mx[0] = fmaxf(mx[0], fabsf(v.x));
-            mx[1] = fmaxf(mx[1], fabsf(v.y));
-            mx[2] = fmaxf(mx[2], fabsf(v.z));
-            mx[3] = fmaxf(mx[3], fabsf(v.w));
-        } else {
-            mx[0] = fmaxf(mx[0], fabsf(*row));
-        }
-    };
-    int r = r0;
-    for (; r + 8 <= r1; r += 8) {
+        for (int u = 0; u < kQuantRound; ++u)
+            x[u] = *reinterpret_cast<const Floats4*>(col + static_cast<size_t>(min(r + u, r1 - 1)) * cols);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) take(r + u);
+        for (int u = 0; u < kQuantRound; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mx[e] = fmaxf(mx[e], fabsf(x[u].v[e]));
     }
-    for (; r < r1; ++r) take(r);
-#pragma unroll
-    for (int e = 0; e < W; ++e) partial[static_cast<size_t>(blockIdx.y) * cols + c + e] = mx[e];
+    *reinterpret_cast<floatx4*>(partial + static_cast<size_t>(blockIdx.y) * stride + 4 * idx) =
+        floatx4{mx[0], mx[1], mx[2], mx[3]};
 }
 
-// scale[c] = absmax / 127 and inv[c] = 1 / scale (0 for a zero column), both
-// correctly rounded (the library is built with IEEE fp32 division). The
-// slice maxima are loaded 16 at a time (max is exact in any order).
-__global__ __launch_bounds__(kThreads) void scale_kernel(int cols, int slices,
+// lround for the range that matters, half away from zero: x + 0.5 less one
+// ulp of it, with x's sign, truncated. The sum reaches the next integer from
+// a fraction of one half up (a tie that rounds to even, or nearer) and from
+// nothing below. The product is rounded to fp32 before anything else reads
+// it (no contraction into the sum), as quant.cpp:23 computes B * inv first.
+__device__ __forceinline__ int quantize_one(float b, float inv) {
+#pragma clang fp contract(off)
+    const float x = b * inv;
+    const float r = x + copysignf(0x1.fffffep-2f, x);
+    return static_cast<int>(fminf(fmaxf(r, -127.0f), 127.0f));
+}
+
+// One slab of rows: scale = absmax / 127 and inv = 1 / scale (0 for a zero
+// column) of the thread's columns, both correctly rounded (the library is
+// built with IEEE fp32 division), from the slices' maxima; then the rows.
+// The first slab writes the scales. Forming them here costs each workgroup
+// `slices` L2 reads a thread and saves a launch.
+__global__ __launch_bounds__(kThreads) void quantize_kernel(int rows, int cols, int span, int stride,
+                                                            int slices, const float* B,
+                                                            const float* partial, float* scale,
+                                                            int8_t* q) {
+    const int idx = blockIdx.x * kThreads + threadIdx.x;
+    if (4 * idx >= stride) return;
+    const int c = column_group(idx, cols);
+    float inv[4];
+    {
+        floatx4 mx{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < slices; s += 16) {
+            floatx4 v[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                v[i] = *reinterpret_cast<const floatx4*>(
+                    partial + static_cast<size_t>(min(s + i, slices - 1)) * stride + 4 * idx);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mx[e] = fmaxf(mx[e], v[i][e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float sc = mx[e] / 127.0f;
+            inv[e] = sc > 0.0f ? 1.0f / sc : 0.0f;
+            if (blockIdx.y == 0) scale[c + e] = sc;
+        }
+    }
+    const int r0 = blockIdx.y * span, r1 = min(rows, r0 + span);
+    for (int r = r0; r < r1; r += kQuantRound) {
+        Floats4 x[kQuantRound];
+#pragma unroll
+        for (int u = 0; u < kQuantRound; ++u)
+            x[u] = *reinterpret_cast<const Floats4*>(B + static_cast<size_t>(min(r + u, r1 - 1)) * cols + c);
+#pragma unroll
+        for (int u = 0; u < kQuantRound; ++u) {
+            if (r + u >= r1) break;
+            uint32_t w = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                w |= (static_cast<uint32_t>(quantize_one(x[u].v[e], inv[e])) & 0xffu) << (8 * e);
+            __builtin_memcpy(q + static_cast<size_t>(r + u) * cols + c, &w, 4);
+        }
+    }
+}
+
+// scale and inv of every column from the slices' maxima, a wave per 16
+// columns: lane 16 p + e takes every fourth slice from p of column e.
+__global__ __launch_bounds__(kThreads) void scale_kernel(int cols, int stride, int slices,
                                                          const float* partial, float* scale,
                                                          float* inv) {
-    const int c = blockIdx.x * kThreads + threadIdx.x;
-    if (c >= cols) return;
+    const int lane = threadIdx.x % kWave, part = lane / 16;
+    const int i = (blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave) * 16 + lane % 16;
+    const int at = min(i, stride - 1);
     float mx = 0.0f;
-    int s = 0;
-    for (; s + 16 <= slices; s += 16) {
+    for (int s = part; s < slices; s += 64) {
         float v[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = partial[static_cast<size_t>(s + i) * cols + c];
+        for (int u = 0; u < 16; ++u)
+            v[u] = partial[static_cast<size_t>(min(s + 4 * u, slices - 1)) * stride + at];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, v[i]);
+        for (int u = 0; u < 16; ++u) mx = fmaxf(mx, v[u]);
     }
-    for (; s < slices; ++s) mx = fmaxf(mx, partial[static_cast<size_t>(s) * cols + c]);
+    mx = max32(max16(mx));
+    if (part != 0 || i >= stride) return;
+    const int c = column_group(i / 4, cols) + i % 4;
     const float sc = mx / 127.0f;
     scale[c] = sc;
     inv[c] = sc > 0.0f ? 1.0f / sc : 0.0f;
 }
 
-// lround for the range that matters: half away from zero, as a float. The
-// product is rounded to fp32 before anything else reads it (no contraction
-// into the subtraction), as quant.cpp:23 computes B * inv first.
-__device__ __forceinline__ float round_half_away(float x) {
-#pragma clang fp contract(off)
-    const float t = truncf(x);
-    return fabsf(x - t) >= 0.5f ? t + copysignf(1.0f, x) : t;
-}
-
-__device__ __forceinline__ int8_t quantize_one(float b, float inv) {
-#pragma clang fp contract(off)
-    const float x = b * inv;
-    const float r = fminf(fmaxf(round_half_away(x), -127.0f), 127.0f);
-    return static_cast<int8_t>(static_cast<int>(r));
-}
-
-// total < 2^31 (checked by the entry point), so int indices suffice. With
-// V4 (cols % 4 == 0, B 16-byte and q 4-byte aligned) a thread takes four
-// consecutive elements of one row: one float4 load and one 32-bit store.
+// The rows of a large matrix, read in address order by the whole grid: four
+// consecutive elements of one row per thread and step (V4: cols % 4 == 0, B
+// 16-byte and q 4-byte aligned), else one.
 template <bool V4>
-__global__ __launch_bounds__(kThreads) void quantize_kernel(int total, int cols, const float* B,
-                                                            const float* inv, int8_t* q) {
+__global__ __launch_bounds__(kThreads) void quantize_flat_kernel(int total, int cols, const float* B,
+                                                                 const float* inv, int8_t* q) {
     if constexpr (V4) {
         const int quads = total / 4;
         for (int i = blockIdx.x * kThreads + threadIdx.x; i < quads; i += gridDim.x * kThreads) {
             const int c = (4 * i) % cols;
             const float4 b = reinterpret_cast<const float4*>(B)[i];
             const float4 s = *reinterpret_cast<const float4*>(inv + c);
-            const uint32_t w = static_cast<uint8_t>(quantize_one(b.x, s.x)) |
-                               static_cast<uint32_t>(static_cast<uint8_t>(quantize_one(b.y, s.y))) << 8 |
-                               static_cast<uint32_t>(static_cast<uint8_t>(quantize_one(b.z, s.z))) << 16 |
-                               static_cast<uint32_t>(static_cast<uint8_t>(quantize_one(b.w, s.w))) << 24;
-            reinterpret_cast<uint32_t*>(q)[i] = w;
+            reinterpret_cast<uint32_t*>(q)[i] =
+                (static_cast<uint32_t>(quantize_one(b.x, s.x)) & 0xffu) |
+                (static_cast<uint32_t>(quantize_one(b.y, s.y)) & 0xffu) << 8 |
+                (static_cast<uint32_t>(quantize_one(b.z, s.z)) & 0xffu) << 16 |
+                (static_cast<uint32_t>(quantize_one(b.w, s.w)) & 0xffu) << 24;
         }
     } else {
         for (int i = blockIdx.x * kThreads + threadIdx.x; i < total; i += gridDim.x * kThreads)
-            q[i] = quantize_one(B[i], inv[i % cols]);
+            q[i] = static_cast<int8_t>(quantize_one(B[i], inv[i % cols]));
     }
+}
+
+// Fewer than four columns: one thread per column does it all.
+__global__ __launch_bounds__(kThreads) void quantize_narrow_kernel(int rows, int cols, const float* B,
+                                                                   int8_t* q, float* scale) {
+    const int c = threadIdx.x;
+    if (c >= cols) return;
+    float mx = 0.0f;
+    for (int r = 0; r < rows; ++r) mx = fmaxf(mx, fabsf(B[static_cast<size_t>(r) * cols + c]));
+    const float sc = mx / 127.0f, inv = sc > 0.0f ? 1.0f / sc : 0.0f;
+    scale[c] = sc;
+    for (int r = 0; r < rows; ++r)
+        q[static_cast<size_t>(r) * cols + c] =
+            static_cast<int8_t>(quantize_one(B[static_cast<size_t>(r) * cols + c], inv));
 }
 
 __global__ __launch_bounds__(kThreads) void dequantize_kernel(int total, int cols,
@@ -246,38 +313,58 @@ void run_fill_zero(float* p, size_t count, hipStream_t stream) {
                        count);
 }
 
+// Past kQuantSmall values (kQuantLarge where the columns' maxima come in few
+// slices) the scales get a launch of their own and the rows are read in
+// address order; up to it the quantising workgroups form them. us, two
+// launches / three: 1000 x 1001 9.5 / 11.2, 300 x 11000 (19 slices) 10.4 /
+// 11.5, 11008 x 257 (256 slices) 19.5 / 15.7, 4096 x 11008 81 / 75.6 (79
+// before).
+constexpr size_t kQuantSmall = size_t{1} << 21, kQuantLarge = size_t{1} << 23;
+constexpr int kQuantFewSlices = 32;
+
 void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale,
                      hipStream_t stream) {
+    if (rows == 0) {
+        run_fill_zero(scale, cols, stream);
+        return;
+    }
+    if (cols < 4) {
+        hipLaunchKernelGGL(quantize_narrow_kernel, dim3(1), dim3(kThreads), 0, stream, rows, cols, B,
+                           q, scale);
+        return;
+    }
+    const int stride = ceil_div(cols, 4) * 4, tiles = ceil_div(stride, 4 * kThreads);
+    // Workgroups towards `per_cu` a CU, each with at least one round of rows.
+    auto slabs = [&](int per_cu, int* span) {
+        const int want = ceil_div(static_cast<long long>(per_cu) * cu_count(), tiles);
+        const int n = std::max(1, std::min(want, ceil_div(rows, kQuantRound)));
+        *span = ceil_div(rows, n);
+        return ceil_div(rows, *span);
+    };
+    const size_t total = static_cast<size_t>(rows) * cols;
+    int span_max = 0, span = 0;
+    int slices = slabs(1, &span_max);
+    const bool large = total > kQuantLarge || (total > kQuantSmall && slices > kQuantFewSlices);
+    if (large) slices = slabs(4, &span_max);
+    const int parts = slabs(2, &span);
+    float* partial = scratch(kQuant, static_cast<size_t>(slices) * stride + stride);
+    hipLaunchKernelGGL(colmax_kernel, dim3(tiles, slices), dim3(kThreads), 0, stream, rows, cols,
+                       span_max, stride, B, partial);
+    if (!large) {
+        hipLaunchKernelGGL(quantize_kernel, dim3(tiles, parts), dim3(kThreads), 0, stream, rows,
+                           cols, span, stride, slices, B, partial, scale, q);
+        return;
+    }
+    float* inv = partial + static_cast<size_t>(slices) * stride;
+    hipLaunchKernelGGL(scale_kernel, dim3(ceil_div(stride, 64)), dim3(kThreads), 0, stream, cols,
+                       stride, slices, partial, scale, inv);
     const bool v4 = cols % 4 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(q) % 4 == 0;
-    // Enough row slices for ~4 workgroups per CU over the column tiles.
-    const int tiles = ceil_div(cols, kThreads * (v4 ? 4 : 1));
-    const int want = ceil_div(4LL * cu_count(), tiles);
-    const int slices = rows ? std::max(1, std::min(want, ceil_div(rows, 16))) : 1;
-    const int span = rows ? ceil_div(rows, slices) : 0;
-    const int used = rows ? ceil_div(rows, span) : 1;
-    float* work = scratch(kQuant, static_cast<size_t>(used) * cols + cols);
-    float* inv = work + static_cast<size_t>(used) * cols;
-    if (rows) {
-        if (v4) {
-            hipLaunchKernelGGL(colmax_kernel<true>, dim3(tiles, used), dim3(kThreads), 0, stream,
-                               rows, cols, span, B, work);
-        } else {
-            hipLaunchKernelGGL(colmax_kernel<false>, dim3(tiles, used), dim3(kThreads), 0, stream,
-                               rows, cols, span, B, work);
-        }
-    } else {
-        run_fill_zero(work, cols, stream);
-    }
-    hipLaunchKernelGGL(scale_kernel, dim3(ceil_div(cols, kThreads)), dim3(kThreads), 0, stream,
-                       cols, used, work, scale, inv);
-    const size_t total = static_cast<size_t>(rows) * cols;
-    if (total == 0) return;
     if (v4) {
-        hipLaunchKernelGGL(quantize_kernel<true>, dim3(grid_for(total / 4)), dim3(kThreads), 0,
+        hipLaunchKernelGGL(quantize_flat_kernel<true>, dim3(grid_for(total / 4)), dim3(kThreads), 0,
                            stream, static_cast<int>(total), cols, B, inv, q);
     } else {
-        hipLaunchKernelGGL(quantize_kernel<false>, dim3(grid_for(total)), dim3(kThreads), 0,
+        hipLaunchKernelGGL(quantize_flat_kernel<false>, dim3(grid_for(total)), dim3(kThreads), 0,
                            stream, static_cast<int>(total), cols, B, inv, q);
     }
 }

@@ -77,3 +77,22 @@ def test_repeat_is_bit_identical():
     a = gpu_quant(B)
     b = gpu_quant(B)
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+# Widths off a group of four and under one, few and many row slices, both
+# sides of the size past which the scales get their own launch.
+@pytest.mark.parametrize("shape", [(1, 1), (5, 3), (17, 4), (33, 5), (400, 7), (700, 66),
+                                   (1000, 1001), (256, 8192), (300, 11000), (3000, 1027)], ids=str)
+def test_ragged_shapes_with_ties_and_zero_columns(shape):
+    rows, cols = shape
+    B = inputs.uniform((rows, cols), -1.0, 1.0, 410 + cols)
+    B[:, 0] = 0.0
+    if cols > 2:
+        # scale 1 exactly: halves are ties, away from zero, up to both ends.
+        B[:, 2] = (np.arange(rows) % 255 - 127) * 0.5
+        B[0, 2] = 127.0
+        B[-1, -1] = -3.0
+    q, s = em.quantize_q8(torch.from_numpy(B).cuda())
+    want_q, want_s = orc.quantize_q8(B)
+    assert np.array_equal(s.cpu().numpy().view(np.uint32), want_s.view(np.uint32))
+    assert np.array_equal(q.cpu().numpy(), want_q)
