@@ -849,6 +849,78 @@ bool split_bf16_preferred(int m, int n, int k) {
 
 namespace {
 
+// 16-row blocks per workgroup, k slices and the slices' rows, and the column
+// tiles that run as two-block tiles in a launch of their own (tail_cols).
+struct Plan {
+    int rb, slices, span, tail_cols;
+};
+
+// More 16-row blocks per workgroup cut how often each weight is widened (the
+// VALU work that paces this kernel); fewer keep more workgroups in flight
+// without a k split and its reduce, round m up by less, and round the grid
+// better (one workgroup per CU at a time).
+//
+// First the largest of 4 / 2 / 1 whose tile grid, weighted by k / 4096 (deeper
+// k holds more work per workgroup), reaches 160 workgroups and, past one per
+// CU, leaves its last round at least 80 % full (70 % with A pre-split into
+// planes), or 4 where its last round can run as two-block tiles: four-block
+// tiles in one slice whose last round is at most half full run that round's
+// column tiles so, one round of twice the workgroups, each about 0.6 of a
+// four-block tile's time, rather than one of half the CUs at a full tile's
+// time (qkv of a 512-row Llama-7B prefill: 384 tiles, 128 of them the last
+// round). Then another of 4 / 3 / 2 / 1 whose estimated time is 6 % or more
+// below that one's. The estimate is a fit over 154 timed shapes (m 20 .. 512,
+// k 1024 .. 11008, widths 1024 .. 22016; 6 % rms off): rounds of the grid,
+// each the chunks of one wave at 0.89 / 1.34 / 1.77 / 2.18 us plus 1.5 us a
+// block (epilogue, first loads), and for slices 2.5 us and the partials'
+// traffic at 3.7 TB/s. With the norm, us with the first rule alone / with
+// both: 4096 x 12288 at m = 40 / 96 / 200 41 / 34, 69 / 50, 83 / 72; 4096 x
+// 22016 at 40 / 96 56 / 48, 83 / 71; 4096 x 6144 at 400 83 / 71; 1024 x 5632
+// at 400 34 / 28.
+//
+// k slices: up to one workgroup per CU, each at least 256 rows deep.
+Plan plan(int m, int n, int k, bool raw) {
+    constexpr double kStepUs[5] = {0.0, 0.89, 1.34, 1.77, 2.18};
+    const int cu = cu_count(), col_tiles = ceil_div(n, kTile);
+    auto tiles = [&](int rb) { return static_cast<long long>(ceil_div(m, 16 * rb)) * col_tiles; };
+    auto fits = [&](int rb) {
+        if (16 * rb > m + 15) return false;
+        const double grid = static_cast<double>(tiles(rb));
+        if (grid * std::max(1.0, k / 4096.0) < 160.0) return false;
+        const double rounds = grid / cu;
+        return rounds <= 1.0 || rounds / std::ceil(rounds) >= (raw ? 0.8 : 0.7);
+    };
+    int first = fits(4) ? 4 : fits(2) ? 2 : 1;
+    if (first != 4 && 64 <= m + 15 && tiles(4) >= cu) {
+        const long long rest = tiles(4) % cu;
+        if (rest > 0 && 2 * rest <= cu && (tiles(4) - rest) % ceil_div(m, 64) == 0) first = 4;
+    }
+    Plan best{0, 1, 0, 0};
+    double best_us = 0.0;
+    for (int i = 0; i <= 4; ++i) {  // `first`, then all
+        const int rb = i == 0 ? first : i;
+        if (16 * rb > m + 15) continue;
+        const int want = static_cast<int>(std::max(1LL, cu / tiles(rb)));
+        Plan p{rb, std::max(1, std::min(want, ceil_div(k, 256))), 0, 0};
+        p.span = ceil_div(ceil_div(k, p.slices), kStep) * kStep;
+        p.slices = ceil_div(k, p.span);
+        auto round_us = [&](int b) { return ceil_div(p.span, kStep) * kStepUs[b] + 1.5 * b; };
+        const long long full = tiles(rb) * p.slices / cu, rest = tiles(rb) * p.slices % cu;
+        double us = 3.2 + (full + (rest > 0)) * round_us(rb);
+        if (p.slices > 1) us += 2.5 + 0.27e-6 * 4.0 * m * n * (2.0 * p.slices + 1.0);
+        if (rb == 4 && p.slices == 1 && full > 0 && rest > 0 && 2 * rest <= cu &&
+            full * cu % ceil_div(m, 64) == 0) {
+            p.tail_cols = col_tiles - static_cast<int>(full * cu / ceil_div(m, 64));
+            us = 3.2 + full * round_us(4) + round_us(2);
+        }
+        if (i == 0 || us < (best.rb == first ? 0.94 : 1.0) * best_us) {
+            best = p;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 // The product, or with pair > 0 the SwiGLU pair (out = a.C, m x pair);
 // false when pair is asked for and the product would need a k split (then
 // nothing is launched). *fused: RoPE was fused.
@@ -859,51 +931,13 @@ bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused)
     const bool raw = !pair && !a.rms_weight && a.k % 8 == 0 &&
                      reinterpret_cast<uintptr_t>(a.A) % 16 == 0;
 
-    // More 16-row blocks per workgroup cut how often each weight is widened
-    // (the VALU work that paces this kernel); fewer keep more workgroups in
-    // flight without a k split and its reduce, and round the grid better
-    // (one workgroup per CU at a time). The largest of 4 / 2 / 1 whose tile
-    // grid, weighted by k / 4096 (deeper k holds more work per workgroup),
-    // reaches 160 workgroups and, past one per CU, leaves its last round at
-    // least 80 % full (70 % with A pre-split into planes, where a workgroup
-    // splits nothing itself and widening weighs more). Over sweeps of
-    // m = 128..1024 and 15 shapes (widths 4096..32000, k 4096 and 11008,
-    // with and without the norm) it averaged 0.6 % above the best of the
-    // three, at most 8 %. At m = 512: 4096^2 takes 2 (55 vs 64 us for 4),
-    // 4096 x 11008 2 (162 vs 177), 4096 x 22016 4 (266 vs 294), 4096 x 32000
-    // 4 (362 vs 408).
     const int col_tiles = ceil_div(a.n, kTile);
-    const double kf = std::max(1.0, a.k / 4096.0);
-    auto fits = [&](int rb) {
-        if (16 * rb > a.m + 15) return false;
-        const double grid = static_cast<double>(ceil_div(a.m, 16 * rb)) * col_tiles;
-        if (grid * kf < 160.0) return false;
-        const double rounds = grid / cu_count();
-        return rounds <= 1.0 || rounds / std::ceil(rounds) >= (raw ? 0.8 : 0.7);
-    };
-    auto tiles = [&](int rb) {
-        return static_cast<long long>(ceil_div(a.m, 16 * rb)) * col_tiles;
-    };
-    int RB = fits(4) ? 4 : fits(2) ? 2 : 1;
-    // Four-block tiles whose last round is at most half full also win when
-    // that round runs as two-block tiles (the tail below), though the rounds
-    // rule above turns them down: 4096 x 11008 at m = 512 131.9 against
-    // 136.9 us (146.3 / 154.2 with the norm; from HBM, 144.9 / 154.6), m =
-    // 1024 244.7 / 249.5; the same bits either way.
-    if (RB != 4 && 64 <= a.m + 15 && tiles(4) >= cu_count()) {
-        const long long cu = cu_count(), g4 = tiles(4), rest = g4 % cu;
-        if (rest > 0 && 2 * rest <= cu && (g4 - rest) % ceil_div(a.m, 64) == 0) RB = 4;
-    }
+    const Plan pl = plan(a.m, a.n, a.k, raw);
+    const int RB = pl.rb, span = pl.span, slices = pl.slices;
     const int row_tiles = ceil_div(a.m, 16 * RB);
     const int m_pad = row_tiles * 16 * RB;
     const int k_pad = ceil_div(a.k, kChunk) * kChunk;
-
-    // k slices up to one workgroup per CU, each at least 256 rows deep.
     const long long blocks = static_cast<long long>(row_tiles) * col_tiles;
-    const int want = static_cast<int>(std::max(1LL, cu_count() / blocks));
-    int slices = std::max(1, std::min(want, ceil_div(a.k, 256)));
-    const int span = ceil_div(ceil_div(a.k, slices), kStep) * kStep;
-    slices = ceil_div(a.k, span);
 
     if (pair && slices > 1) return false;
 
@@ -964,20 +998,7 @@ bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused)
                       rope->dim % 4 == 0 && rope->kv_dim % 4 == 0 &&
                       a.n == rope->dim + 2 * rope->kv_dim;
     if (fuse) p.rope = *rope;
-    // A product in one slice whose four-block tiles leave a last round at
-    // most half full runs that round's column tiles as two-block tiles: one
-    // round of twice the workgroups, each about 0.7 of a four-block tile's
-    // time (widening shared by half the rows), rather than one of half the
-    // CUs at a full tile's time. Same arithmetic per element, so the same
-    // bits. qkv of a 512-row Llama-7B prefill: 384 tiles, 128 of them the
-    // last round.
-    int tail_cols = 0;
-    if (RB == 4 && slices == 1) {
-        const long long cu = cu_count();
-        const long long full = blocks / cu * cu, rest = blocks - full;
-        if (full > 0 && rest > 0 && 2 * rest <= cu && full % row_tiles == 0)
-            tail_cols = col_tiles - static_cast<int>(full / row_tiles);
-    }
+    const int tail_cols = pl.tail_cols;
     if (tail_cols > 0) {
         p.col_tiles = col_tiles - tail_cols;
         launch<4>(p, row_tiles * p.col_tiles, raw, a.stream);
@@ -993,6 +1014,7 @@ bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused)
     const int total = static_cast<int>(blocks) * slices;
     switch (RB) {
         case 1: launch<1>(p, total, raw, a.stream); break;
+        case 3: launch<3>(p, total, raw, a.stream); break;
         case 4: launch<4>(p, total, raw, a.stream); break;
         default: launch<2>(p, total, raw, a.stream); break;
     }
