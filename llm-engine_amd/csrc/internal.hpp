@@ -163,7 +163,9 @@ struct RopeFuse {
 // With rope, and when the product needs no k split (it writes C directly):
 // q is stored rotated, k rotated into kc and v into vc (not into C), with
 // rope_cache_kernel's arithmetic; returns true. Otherwise C as usual, false.
-bool run_split_bf16(const MatmulArgs& a, const RopeFuse* rope = nullptr);
+// whole: k slices are chosen as for a call with rope (with and without rope
+// then give the same bits).
+bool run_split_bf16(const MatmulArgs& a, const RopeFuse* rope = nullptr, bool whole = false);
 // The forward pass's w13 with its SwiGLU: B (k x 2 hidden) holds gates then
 // ups, a.C is hidden wide and gets silu(gate) * up, the bits of the product
 // followed by swiglu_kernel. False, nothing launched, when the shape is not

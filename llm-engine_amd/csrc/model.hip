@@ -50,12 +50,21 @@ namespace {
 // every load issue before the stores. With ssq (dim % 64 == 0, one row) it
 // also writes the sum of squares of each 64 values, for the first layer's
 // qkv GEMV norm: 16 lanes' float4s, added by a fixed butterfly. Token ids
-// were range-checked on the host.
+// were range-checked on the host. With pos_out, `feed` is the host's own
+// pinned copy, read here by system-scope loads (one token: two words over the
+// bus, against a copy node before this launch), and the position goes on to
+// device memory for the step's other kernels.
 __global__ __launch_bounds__(kThreads) void embed_kernel(int dim, const int* __restrict__ feed,
+                                                         int* __restrict__ pos_out,
                                                          const float* __restrict__ table,
                                                          float* __restrict__ x,
                                                          float* __restrict__ ssq) {
-    const std::size_t src = static_cast<std::size_t>(feed[1 + blockIdx.y]) * dim;
+    auto word = [&](int i) {
+        return pos_out ? __hip_atomic_load(feed + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                       : feed[i];
+    };
+    if (pos_out && blockIdx.x == 0 && threadIdx.x == 0) *pos_out = word(0);
+    const std::size_t src = static_cast<std::size_t>(word(1 + blockIdx.y)) * dim;
     const std::size_t dst = static_cast<std::size_t>(blockIdx.y) * dim;
     const int j = blockIdx.x * kThreads + threadIdx.x;
     if (dim % 4 == 0) {
@@ -185,13 +194,22 @@ struct Stream {
     }
 };
 
-// Pinned host memory, so the feed and logits copies can be graph nodes.
+// Pinned host memory that kernels read and write in place (dev: its address
+// for them), so a one-token step needs no copy nodes: each cost its own
+// 3 to 5 us and a launch gap.
 template <class T>
 struct Pinned {
     T* p = nullptr;
+    T* dev = nullptr;
     explicit Pinned(std::size_t count) {
         check(hipHostMalloc(reinterpret_cast<void**>(&p), count * sizeof(T), hipHostMallocDefault),
               "alloc pinned");
+        const hipError_t err =
+            hipHostGetDevicePointer(reinterpret_cast<void**>(&dev), p, 0);
+        if (err != hipSuccess) {
+            (void)hipHostFree(p);
+            check(err, "map pinned");
+        }
     }
     Pinned(const Pinned&) = delete;
     Pinned& operator=(const Pinned&) = delete;
@@ -278,7 +296,7 @@ private:
     em_model_config cfg_;
     bool q8_;
     AttnShape shape_;
-    Buf<float> emb_, rms_final_, rope_cos_, rope_sin_, logits_dev_;
+    Buf<float> emb_, rms_final_, rope_cos_, rope_sin_;
     Proj wcls_;
     std::vector<LayerDev> layers_;
     std::size_t filled_ = 0;
@@ -374,7 +392,6 @@ void Model::init_runtime() {
     upload(rope_cos_, cs.data(), cs.size());
     upload(rope_sin_, sn.data(), sn.size());
 
-    logits_dev_.alloc(V);
     feed_dev_.alloc(c.seq_len + 1);
     use_ssq_ = D % kSsqChunk == 0 && D / kSsqChunk <= 256;
     if (use_ssq_) ssq_.alloc(D / kSsqChunk);
@@ -825,7 +842,7 @@ bool Model::qkv_exact_split(int n, LayerDev& L, bool* roped) {
     const RopeFuse r{feed_dev_.p, rope_cos_.p, rope_sin_.p, L.kcache.p, L.vcache.p,
                      static_cast<int>(cfg_.dim), static_cast<int>(shape_.kv_stride),
                      shape_.head_size};
-    *roped = run_split_bf16(a, rope_fusion_ ? &r : nullptr);
+    *roped = run_split_bf16(a, rope_fusion_ ? &r : nullptr, true);
     check(hipGetLastError(), "launch");
     return true;
 }
@@ -894,9 +911,12 @@ void Model::enqueue(int n) {
     const int D = static_cast<int>(cfg_.dim), H = static_cast<int>(cfg_.hidden_dim);
     const int KV = static_cast<int>(shape_.kv_stride), hs = shape_.head_size;
     const int qkv_cols = static_cast<int>(shape_.q_stride);
-    check(hipMemcpyAsync(feed_dev_.p, feed_host_.p, (n + 1) * sizeof(int), hipMemcpyHostToDevice,
-                         stream_),
-          "upload feed");
+    // One token is read from the host's copy by embed_kernel; a prompt's are
+    // uploaded.
+    if (n > 1)
+        check(hipMemcpyAsync(feed_dev_.p, feed_host_.p, (n + 1) * sizeof(int),
+                             hipMemcpyHostToDevice, stream_),
+              "upload feed");
     // One-token steps over strip copies: each product is one em_matmul_q8
     // call (the norm formed inside it). Other one-token steps hand the norm
     // GEMVs the sums of squares of x from whichever kernel last wrote x
@@ -904,7 +924,8 @@ void Model::enqueue(int n) {
     const bool strip_step = n == 1 && strips_;
     bool have_ssq = n == 1 && use_ssq_ && !strip_step;
     hipLaunchKernelGGL(embed_kernel, dim3(ceil_div(ceil_div(D, 4), kThreads), n), dim3(kThreads), 0,
-                       stream_, D, feed_dev_.p, emb_.p, x_.p, have_ssq ? ssq_.p : nullptr);
+                       stream_, D, n > 1 ? feed_dev_.p : feed_host_.dev,
+                       n > 1 ? nullptr : feed_dev_.p, emb_.p, x_.p, have_ssq ? ssq_.p : nullptr);
     const int rope_threads = D / 2 + KV / 2 + KV;
     const int swiglu_blocks = std::min(ceil_div(static_cast<long long>(n) * H, kThreads), 4096);
     for (LayerDev& L : layers_) {
@@ -974,22 +995,20 @@ void Model::enqueue(int n) {
             have_ssq = false;
         }
     }
-    // Only the last row's logits are returned.
+    // Only the last row's logits are returned, written by the classifier's
+    // kernel straight into the host's pinned buffer.
     const float* x_last = x_.p + static_cast<std::size_t>(n - 1) * D;
     if (have_ssq) {
         const MatmulArgs a =
-            gemv_args(1, x_last, wcls_, logits_dev_.p, rms_final_.p, false, ssq_.p);
+            gemv_args(1, x_last, wcls_, logits_host_.dev, rms_final_.p, false, ssq_.p);
         if (q8_) {
             run_skinny<int8_t>(a);
         } else {
             run_skinny<float>(a);
         }
     } else {
-        project(1, x_last, wcls_, logits_dev_.p, rms_final_.p, false);
+        project(1, x_last, wcls_, logits_host_.dev, rms_final_.p, false);
     }
-    check(hipMemcpyAsync(logits_host_.p, logits_dev_.p, cfg_.vocab_size * sizeof(float),
-                         hipMemcpyDeviceToHost, stream_),
-          "download logits");
     check(hipGetLastError(), "launch");
 }
 

@@ -878,8 +878,11 @@ struct Plan {
 // 22016 at 40 / 96 56 / 48, 83 / 71; 4096 x 6144 at 400 83 / 71; 1024 x 5632
 // at 400 34 / 28.
 //
-// k slices: up to one workgroup per CU, each at least 256 rows deep.
-Plan plan(int m, int n, int k, bool raw) {
+// k slices: up to one workgroup per CU, each at least 256 rows deep. `whole`:
+// a call whose epilogue would do a following kernel's work if k were whole;
+// slices then cost that kernel too (the forward pass's RoPE and cache write,
+// 3 us and two passes over the product at 2.5 TB/s).
+Plan plan(int m, int n, int k, bool raw, bool whole) {
     constexpr double kStepUs[5] = {0.0, 0.89, 1.34, 1.77, 2.18};
     const int cu = cu_count(), col_tiles = ceil_div(n, kTile);
     auto tiles = [&](int rb) { return static_cast<long long>(ceil_div(m, 16 * rb)) * col_tiles; };
@@ -908,6 +911,7 @@ Plan plan(int m, int n, int k, bool raw) {
         const long long full = tiles(rb) * p.slices / cu, rest = tiles(rb) * p.slices % cu;
         double us = 3.2 + (full + (rest > 0)) * round_us(rb);
         if (p.slices > 1) us += 2.5 + 0.27e-6 * 4.0 * m * n * (2.0 * p.slices + 1.0);
+        if (p.slices > 1 && whole) us += 3.0 + 0.4e-6 * 8.0 * m * n;
         if (rb == 4 && p.slices == 1 && full > 0 && rest > 0 && 2 * rest <= cu &&
             full * cu % ceil_div(m, 64) == 0) {
             p.tail_cols = col_tiles - static_cast<int>(full * cu / ceil_div(m, 64));
@@ -924,7 +928,7 @@ Plan plan(int m, int n, int k, bool raw) {
 // The product, or with pair > 0 the SwiGLU pair (out = a.C, m x pair);
 // false when pair is asked for and the product would need a k split (then
 // nothing is launched). *fused: RoPE was fused.
-bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused) {
+bool split_run(const MatmulArgs& a, const RopeFuse* rope, bool whole, int pair, bool* fused) {
     // Without a norm, the kernel splits A itself, chunk by chunk (needs whole
     // 8-value groups and 16-byte rows); otherwise a pre-pass writes the three
     // planes with the norm fused. The SwiGLU pair always reads the planes.
@@ -932,7 +936,7 @@ bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused)
                      reinterpret_cast<uintptr_t>(a.A) % 16 == 0;
 
     const int col_tiles = ceil_div(a.n, kTile);
-    const Plan pl = plan(a.m, a.n, a.k, raw);
+    const Plan pl = plan(a.m, a.n, a.k, raw, whole);
     const int RB = pl.rb, span = pl.span, slices = pl.slices;
     const int row_tiles = ceil_div(a.m, 16 * RB);
     const int m_pad = row_tiles * 16 * RB;
@@ -1025,9 +1029,9 @@ bool split_run(const MatmulArgs& a, const RopeFuse* rope, int pair, bool* fused)
 
 }  // namespace
 
-bool run_split_bf16(const MatmulArgs& a, const RopeFuse* rope) {
+bool run_split_bf16(const MatmulArgs& a, const RopeFuse* rope, bool whole) {
     bool fused = false;
-    split_run(a, rope, 0, &fused);
+    split_run(a, rope, whole, 0, &fused);
     return fused;
 }
 
@@ -1039,7 +1043,7 @@ bool split_bf16_swiglu_supported(const MatmulArgs& a, int hidden) {
 bool run_split_bf16_swiglu(const MatmulArgs& a, int hidden) {
     if (!split_bf16_swiglu_supported(a, hidden)) return false;
     bool fused = false;
-    return split_run(a, nullptr, hidden, &fused);
+    return split_run(a, nullptr, false, hidden, &fused);
 }
 
 }  // namespace em
