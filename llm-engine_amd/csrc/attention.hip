@@ -303,8 +303,13 @@ __device__ void merge_chunks(const AttnArgs& a, int i, int h0, int G, int n, flo
 // (the workgroup of the first head group of each kv head) and takes that
 // position in slot 0 after its loop, from LDS: no workgroup reads a cache
 // row written in the same launch.
-template <int G, int LPP, int F, bool ROPE = false>
-__global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
+//
+// PIPE: the next round's keys are loaded once this round's are used, beside
+// its softmax and values, and its values after them, in the same registers
+// (up to four heads keep to 128, so four workgroups share a CU). split_pipes
+// says where.
+template <int G, int LPP, int F, bool ROPE = false, bool PIPE = false>
+__global__ __launch_bounds__(kThreads, PIPE && G <= 4 ? 4 : 1) void attn_split_kernel(AttnArgs a) {
     constexpr int NS = kThreads / LPP;
     constexpr int MC = G > 1 ? kSplitMinChunkGrouped : kSplitMinChunk;  // min_chunk of the shape
     constexpr int PP = MC / NS < kRoundPerSlot ? (MC / NS > 0 ? MC / NS : 1) : kRoundPerSlot;
@@ -344,17 +349,13 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
     // before the ROPE query is formed measured 1 us slower at ctx 512: the
     // query's loads then wait behind the whole chunk's.)
     floatx4 kv[PP][F], vv[PP][F];
-    auto load_round = [&](int b0) {
+    auto load_round = [&](floatx4 (&x)[PP][F], const float* base, int b0) {
 #pragma unroll
         for (int pp = 0; pp < PP; ++pp) {
             const int t = min(b0 + slot + pp * NS, loop_len - 1);
-            const floatx4* kr = reinterpret_cast<const floatx4*>(kbase + static_cast<std::size_t>(t) * a.kv_stride);
-            const floatx4* vr = reinterpret_cast<const floatx4*>(vbase + static_cast<std::size_t>(t) * a.kv_stride);
+            const floatx4* r = reinterpret_cast<const floatx4*>(base + static_cast<std::size_t>(t) * a.kv_stride);
 #pragma unroll
-            for (int f = 0; f < F; ++f) {
-                kv[pp][f] = kr[dcol[f]];
-                vv[pp][f] = vr[dcol[f]];
-            }
+            for (int f = 0; f < F; ++f) x[pp][f] = r[dcol[f]];
         }
     };
 
@@ -420,8 +421,16 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
         for (int f = 0; f < F; ++f) o[g][f] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
+    if (PIPE && loop_len > 0) {
+        load_round(kv, kbase, 0);
+        load_round(vv, vbase, 0);
+    }
     for (int b0 = 0; b0 < loop_len; b0 += ROUND) {
-        load_round(b0);
+        const bool more = PIPE && b0 + ROUND < loop_len;
+        if constexpr (!PIPE) {
+            load_round(kv, kbase, b0);
+            load_round(vv, vbase, b0);
+        }
         float sc[G][PP];
 #pragma unroll
         for (int pp = 0; pp < PP; ++pp) {
@@ -439,6 +448,7 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
                 sc[g][pp] = valid ? dot * scale : -INFINITY;
             }
         }
+        if (more) load_round(kv, kbase, b0 + ROUND);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             float mb = sc[g][0];
@@ -459,6 +469,7 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(AttnArgs a) {
             }
             m[g] = mn;
         }
+        if (more) load_round(vv, vbase, b0 + ROUND);
     }
 
     if (own_pos && slot == 0) {
@@ -1270,13 +1281,35 @@ void launch_merge(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t s
                        (slots * dpw * 4 + 2 * slots) * sizeof(float), stream, a);
 }
 
+// Where overlapping a chunk's rounds pays (us, apart / overlapped): four rows
+// of 32 heads of 64 at context 4096 / 9000 38 / 32, 95 / 73, of 128 at 9000
+// 135 / 121, of 32 on 8 kv heads of 128 82 / 77; one row of 32 heads of 64 at
+// 9000 37.7 / 33.5. Not for one row of two or four heads of 128 a workgroup,
+// whose four-deep grid already overlaps (8 kv heads at 9000 / 16384 28.2 /
+// 29.6, 37.8 / 40.9), nor past 128 dims, where it spills.
+template <int G, int LPP>
+constexpr bool split_pipes(int rows) {
+    return LPP <= 32 && (rows > 1 || G == 1 || G == 8 || LPP <= 16);
+}
+
 // Rows of fewer than a.merge_from chunks are left for the caller to merge;
 // no merge launches when no row can have that many.
 template <int G, int LPP, int F, bool ROPE>
 void launch_split(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t stream) {
     const dim3 grid(s.n_heads / G, rows, a.splits);
-    hipLaunchKernelGGL((attn_split_kernel<G, LPP, F, ROPE>), grid, dim3(kThreads),
-                       split_lds(s, ROPE, a.merge_count != nullptr), stream, a);
+    const std::size_t lds = split_lds(s, ROPE, a.merge_count != nullptr);
+    bool piped = false;
+    if constexpr (split_pipes<G, LPP>(ROPE ? 1 : 2)) {
+        piped = split_pipes<G, LPP>(rows);
+        if (piped)
+            hipLaunchKernelGGL((attn_split_kernel<G, LPP, F, ROPE, true>), grid, dim3(kThreads), lds,
+                               stream, a);
+    }
+    if constexpr (!split_pipes<G, LPP>(1)) {
+        if (!piped)
+            hipLaunchKernelGGL((attn_split_kernel<G, LPP, F, ROPE>), grid, dim3(kThreads), lds, stream,
+                               a);
+    }
     if (a.merge_count) return;  // the kernel merges its own rows
     if (a.splits < a.merge_from) return;  // e.g. one chunk per row: written directly
     launch_merge(s, a, rows, stream);
