@@ -191,6 +191,7 @@ struct AttnArgs {
     int n_heads, head_size, group, seq_len, splits, chunk_cap, rows;
     int min_chunk;   // split_chunk's least chunk for this shape
     int whole;       // contexts of up to this many positions are one chunk
+    int group_chunk_min;  // grouped tile kernel: least positions per chunk (0: not it)
     int merge_from;  // the merge kernel takes rows of at least this many chunks (>= 2)
     int tile_chunk;  // tile kernel split over the context: positions per chunk (0: no split)
     int q_stride, kv_stride, out_stride;
@@ -215,6 +216,13 @@ struct AttnArgs {
     // zero between calls), not by a merge launch.
     unsigned* merge_count;
 };
+
+// Positions per chunk of the grouped tile kernel for a call whose last row has
+// n_ctx: whole 16-position blocks.
+__device__ __forceinline__ int group_chunk(int n_ctx, int splits, int least) {
+    const int c = (n_ctx + splits - 1) / splits;
+    return ((c > least ? c : least) + 15) / 16 * 16;
+}
 
 // Lanes per key row: hs4 rounded up to a power of two, at most one wave.
 __device__ __forceinline__ int lanes_per_row(int n) {
@@ -583,8 +591,9 @@ __global__ __launch_bounds__(kThreads) void attn_merge_kernel(AttnArgs a) {
     const int h = blockIdx.x / groups, d0 = (blockIdx.x % groups) * dpw;
     const int i = blockIdx.y;
     const int n_ctx = *a.pos + i + 1;
-    const int chunk = a.tile_chunk       ? a.tile_chunk
-                      : n_ctx <= a.whole ? n_ctx
+    const int chunk = a.tile_chunk         ? a.tile_chunk
+                      : a.group_chunk_min  ? group_chunk(*a.pos + a.rows, a.splits, a.group_chunk_min)
+                      : n_ctx <= a.whole   ? n_ctx
                                          : split_chunk(n_ctx, a.splits, a.min_chunk);
     const int n = (n_ctx + chunk - 1) / chunk;
     if (n < a.merge_from) return;  // one chunk: written by the split kernel; few: by their consumer
@@ -758,21 +767,25 @@ __device__ __forceinline__ void load_run(const float* src, float* dst) {
 }
 
 constexpr int kTileWaves = 4;
+constexpr int kGroupChunkMin = 64, kGroupWorkgroups = 512;
 
 // One wave's online softmax over positions [first, wlast] (both ends of
-// whole 16-position blocks) for the 16 queries r0 + j of head h: max m, this
-// lane's part l of the sum, unnormalised output o. `last` is the last
-// position that may be read.
-template <int E>
-__device__ __forceinline__ void tile_wave(const AttnArgs& a, int h, int r0, int last, int first,
-                                          int wlast, float& m, float& l, floatx4 (&o)[E]) {
+// whole 16-position blocks) for 16 queries on the keys and values of one kv
+// head; this lane's is row `row` of query head `h` (any of the kv head's):
+// max m, this lane's part l of the sum, unnormalised output o. `last` is the
+// last position that may be read. FINE keeps the chains of additions as short
+// as the split kernel's: a score is a tree over four-product sums, the output
+// a sum over blocks of two eight-product sums each.
+template <int E, bool FINE = false>
+__device__ __forceinline__ void tile_wave(const AttnArgs& a, int kvh, int h, int row, int last,
+                                          int first, int wlast, float& m, float& l,
+                                          floatx4 (&o)[E]) {
     constexpr int HS = 16 * E, Q4 = 4 * E;
     constexpr int KB = 16;  // positions per block
     const int lane = threadIdx.x % kWave, g = lane >> 4, j = lane & 15;
-    const int row = min(r0 + j, a.rows - 1);  // rows past the call: computed, not stored
-    const int pq = *a.pos + row;              // this lane's query position
-    const float* kbase = a.kc + static_cast<std::size_t>((h / a.group) * HS);
-    const float* vbase = a.vc + static_cast<std::size_t>((h / a.group) * HS);
+    const int pq = *a.pos + row;  // this lane's query position
+    const float* kbase = a.kc + static_cast<std::size_t>(kvh * HS);
+    const float* vbase = a.vc + static_cast<std::size_t>(kvh * HS);
 
     float q[Q4];
     load_run<Q4>(a.q + static_cast<std::size_t>(row) * a.q_stride + static_cast<std::size_t>(h) * HS + Q4 * g, q);
@@ -804,8 +817,27 @@ __device__ __forceinline__ void tile_wave(const AttnArgs& a, int h, int r0, int 
         floatx4 sacc[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) sacc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (FINE) {
+            floatx4 part[E];
 #pragma unroll
-        for (int u = 0; u < Q4; ++u) sacc[u & 3] = mfma16x16x4(b.k[u / 4][u % 4], q[u], sacc[u & 3]);
+            for (int u = 0; u < E; ++u) {
+                floatx4 d[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    d[c] = mfma16x16x4(b.k[u][c], q[4 * u + c], floatx4{0.f, 0.f, 0.f, 0.f});
+                part[u] = (d[0] + d[1]) + (d[2] + d[3]);
+            }
+#pragma unroll
+            for (int n = 1; n < E; n *= 2) {
+#pragma unroll
+                for (int u = 0; u + n < E; u += 2 * n) part[u] += part[u + n];
+            }
+            sacc[0] = part[0];
+        } else {
+#pragma unroll
+            for (int u = 0; u < Q4; ++u)
+                sacc[u & 3] = mfma16x16x4(b.k[u / 4][u % 4], q[u], sacc[u & 3]);
+        }
         float sv[4];
         float mb = -INFINITY;
 #pragma unroll
@@ -823,14 +855,28 @@ __device__ __forceinline__ void tile_wave(const AttnArgs& a, int h, int r0, int 
         const bool none = mn == -INFINITY;
         const float alpha = none ? 1.0f : expf(m - mn);
         l *= alpha;
-#pragma unroll
-        for (int c = 0; c < E; ++c) o[c] *= alpha;
+        float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float p = none ? 0.0f : expf(sv[r] - mn);
-            l += p;
+            p[r] = none ? 0.0f : expf(sv[r] - mn);
+            l += p[r];
+        }
+        if constexpr (FINE) {
 #pragma unroll
-            for (int c = 0; c < E; ++c) o[c] = mfma16x16x4(b.v[r][c], p, o[c]);
+            for (int c = 0; c < E; ++c) {
+                floatx4 d0 = mfma16x16x4(b.v[0][c], p[0], floatx4{0.f, 0.f, 0.f, 0.f});
+                floatx4 d1 = mfma16x16x4(b.v[2][c], p[2], floatx4{0.f, 0.f, 0.f, 0.f});
+                d0 = mfma16x16x4(b.v[1][c], p[1], d0);
+                d1 = mfma16x16x4(b.v[3][c], p[3], d1);
+                o[c] = o[c] * alpha + (d0 + d1);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < E; ++c) o[c] *= alpha;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < E; ++c) o[c] = mfma16x16x4(b.v[r][c], p[r], o[c]);
         }
         m = mn;
     };
@@ -848,27 +894,66 @@ __device__ __forceinline__ void tile_wave(const AttnArgs& a, int h, int r0, int 
     }
 }
 
-// The result of query r0 + j over positions from lo = cz * tile_chunk on:
-// max M, whole sum l, unnormalised output. Split: a query whose context
-// spans more than one chunk leaves this chunk's state for the merge kernel;
-// one whose context fits chunk 0 is written here, as the split kernel writes
-// it. run(u, f) is the float4 of f * the output at head dims run_at(u) ..
-// + 3, u < E.
-template <int E, class At, class Run>
-__device__ __forceinline__ void tile_store(const AttnArgs& a, int h, int r0, int cz, float M,
-                                           float l, At run_at, Run run) {
+// tile_wave position by position without matrix products, where a masked
+// position (one past the lane's query) must not reach the output even as a
+// product with zero: a value that is not finite. The output in tile_wave's
+// layout: head dim 4E g + x in o[x % E][x / E].
+template <int E>
+__device__ void tile_wave_plain(const AttnArgs& a, int kvh, int h, int row, int last, int first,
+                                int wlast, float& m, float& l, floatx4 (&o)[E]) {
     constexpr int HS = 16 * E;
-    const int lane = threadIdx.x % kWave, g = lane >> 4, j = lane & 15;
-    const int pq = *a.pos + min(r0 + j, a.rows - 1), lo = cz * a.tile_chunk;
-    if (r0 + j < a.rows && a.tile_chunk && pq >= a.tile_chunk && lo <= pq) {
-        const std::size_t b = (static_cast<std::size_t>(r0 + j) * a.n_heads + h) * a.splits + cz;
+    const int g = (threadIdx.x % kWave) >> 4, pq = *a.pos + row;
+    const floatx4* q = reinterpret_cast<const floatx4*>(
+        a.q + static_cast<std::size_t>(row) * a.q_stride + static_cast<std::size_t>(h) * HS + 4 * E * g);
+    const std::size_t base = static_cast<std::size_t>(kvh * HS) + 4 * E * g;
+    const float scale = 1.0f / sqrtf(static_cast<float>(HS));
+    m = -INFINITY;
+    l = 0.0f;
+    for (int u = 0; u < E; ++u) o[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = first; t <= min(wlast, last); ++t) {
+        const std::size_t off = base + static_cast<std::size_t>(t) * a.kv_stride;
+        const floatx4* k = reinterpret_cast<const floatx4*>(a.kc + off);
+        const floatx4* v = reinterpret_cast<const floatx4*>(a.vc + off);
+        float x = 0.0f;
+        for (int u = 0; u < E; ++u) {
+            const floatx4 y = q[u] * k[u];
+            x += (y[0] + y[1]) + (y[2] + y[3]);
+        }
+        x = sum32(sum16(x)) * scale;
+        if (t > pq) continue;
+        const float mn = fmaxf(m, x), alpha = m == mn ? 1.0f : expf(m - mn), p = expf(x - mn);
+        l = l * alpha + p;
+#pragma unroll
+        for (int x = 0; x < 4 * E; ++x)
+            o[x % E][x / E] = o[x % E][x / E] * alpha + p * v[x / 4][x % 4];
+        m = mn;
+    }
+    // Each of a query's four lanes has the whole sum; the caller adds them.
+    if (g) l = 0.0f;
+}
+
+// The result of row `row` of head h over positions from lo = cz * chunk on
+// (chunk 0: the whole context): max M, whole sum l, unnormalised output.
+// Split: a query whose context spans more than one chunk leaves this chunk's
+// state for the merge kernel; one whose context fits chunk 0 is written here,
+// as the split kernel writes it. run(u, f) is the float4 of f * the output at
+// head dims run_at(u) .. + 3, u < E. Rows past the call store nothing.
+template <int E, class At, class Run>
+__device__ __forceinline__ void tile_store(const AttnArgs& a, int h, int row, int cz, int chunk,
+                                           float M, float l, At run_at, Run run) {
+    constexpr int HS = 16 * E;
+    const int g = (threadIdx.x % kWave) >> 4;
+    if (row >= a.rows) return;
+    const int pq = *a.pos + row, lo = cz * chunk;
+    if (chunk && pq >= chunk && lo <= pq) {
+        const std::size_t b = (static_cast<std::size_t>(row) * a.n_heads + h) * a.splits + cz;
 #pragma unroll
         for (int u = 0; u < E; ++u)
             *reinterpret_cast<floatx4*>(a.part_o + b * HS + run_at(u)) = run(u, 1.0f);
         if (g == 0) a.part_ml[b] = make_float2(M, l);
-    } else if (r0 + j < a.rows && cz == 0 && (a.tile_chunk == 0 || pq < a.tile_chunk)) {
+    } else if (cz == 0 && (chunk == 0 || pq < chunk)) {
         const float inv = 1.0f / l;
-        float* dst = a.out + static_cast<std::size_t>(r0 + j) * a.out_stride +
+        float* dst = a.out + static_cast<std::size_t>(row) * a.out_stride +
                      static_cast<std::size_t>(h) * HS;
 #pragma unroll
         for (int u = 0; u < E; ++u) *reinterpret_cast<floatx4*>(dst + run_at(u)) = run(u, inv);
@@ -877,47 +962,48 @@ __device__ __forceinline__ void tile_store(const AttnArgs& a, int h, int r0, int
 
 // tile_store of tile_wave's layout: o[c][r] is head dim E (4g + r) + c.
 template <int E>
-__device__ __forceinline__ void tile_store_wave(const AttnArgs& a, int h, int r0, int cz, float M,
-                                                float l, const floatx4 (&o)[E]) {
+__device__ __forceinline__ void tile_store_wave(const AttnArgs& a, int h, int row, int cz, int chunk,
+                                                float M, float l, const floatx4 (&o)[E]) {
     float flat[4 * E];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int c = 0; c < E; ++c) flat[E * r + c] = o[c][r];
     const int g = (threadIdx.x % kWave) >> 4;
-    tile_store<E>(a, h, r0, cz, M, l, [&](int u) { return 4 * E * g + 4 * u; },
+    tile_store<E>(a, h, row, cz, chunk, M, l, [&](int u) { return 4 * E * g + 4 * u; },
                   [&](int u, float f) {
                       return floatx4{flat[4 * u] * f, flat[4 * u + 1] * f, flat[4 * u + 2] * f,
                                      flat[4 * u + 3] * f};
                   });
 }
 
-template <int E>
-__global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs a) {
+// A tile workgroup: its waves take quarters of the blocks of positions [lo,
+// hi] (lo a multiple of 16) for the same 16 queries, then merge in LDS.
+template <int E, bool FINE = false>
+__device__ __forceinline__ void tile_block(const AttnArgs& a, int kvh, int h, int row, int last,
+                                           int lo, int hi, int cz, int chunk) {
     constexpr int KB = 16;  // positions per block
     __shared__ float ms[kTileWaves][kWave], ls[kTileWaves][kWave];
     __shared__ floatx4 os[kTileWaves][E][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // Row tiles in reverse: the longest (causal) start first and the short
-    // ones fill in behind them.
-    const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kTileRows;
-    const int last = *a.pos + min(r0 + kTileRows - 1, a.rows - 1);  // the tile's last position
-    // Split over the context: this workgroup takes positions [lo, hi] of
-    // chunk blockIdx.z (none past last: the grid is sized for seq_len).
-    const int cz = blockIdx.z;
-    const int lo = cz * a.tile_chunk;
-    if (lo > last) return;
-    const int hi = a.tile_chunk ? min(last, lo + a.tile_chunk - 1) : last;
-
     // This wave's blocks: [nb * w / 4, nb * (w + 1) / 4) of the nb blocks
-    // from lo (a multiple of 16) through hi.
+    // from lo through hi.
     const int b0i = lo / KB, nb = hi / KB + 1 - b0i;
     const int first = KB * (b0i + nb * wave / kTileWaves);
     const int wlast = KB * (b0i + nb * (wave + 1) / kTileWaves) - 1;  // < first: no blocks
     float m, l;
     floatx4 o[E];
-    tile_wave<E>(a, h, r0, last, first, wlast, m, l, o);
+    tile_wave<E, FINE>(a, kvh, h, min(row, a.rows - 1), last, first, wlast, m, l, o);
+    if constexpr (FINE) {
+        bool bad = !(l < INFINITY);
+#pragma unroll
+        for (int c = 0; c < E; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad |= !(fabsf(o[c][e]) < INFINITY);
+        if (__ballot(bad))
+            tile_wave_plain<E>(a, kvh, h, min(row, a.rows - 1), last, first, wlast, m, l, o);
+    }
 
     // Merge the waves in order: lane l of every wave holds query j's state.
     ms[wave][lane] = m;
@@ -947,7 +1033,43 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs 
     // the xor pairs add them in the same order in every lane.
     l += __shfl_xor(l, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
-    tile_store_wave<E>(a, h, r0, cz, M, l, o);
+    tile_store_wave<E>(a, h, row, cz, chunk, M, l, o);
+}
+
+template <int E>
+__global__ __launch_bounds__(kTileWaves * kWave) void attn_tile_kernel(AttnArgs a) {
+    // Row tiles in reverse: the longest (causal) start first and the short
+    // ones fill in behind them.
+    const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kTileRows;
+    const int last = *a.pos + min(r0 + kTileRows - 1, a.rows - 1);  // the tile's last position
+    // Split over the context: this workgroup takes positions [lo, hi] of
+    // chunk blockIdx.z (none past last: the grid is sized for seq_len).
+    const int cz = blockIdx.z, lo = cz * a.tile_chunk;
+    if (lo > last) return;
+    const int hi = a.tile_chunk ? min(last, lo + a.tile_chunk - 1) : last;
+    tile_block<E>(a, h / a.group, h, r0 + static_cast<int>(threadIdx.x % 16), last, lo, hi, cz,
+                  a.tile_chunk);
+}
+
+// A few rows of grouped heads: workgroup (kv head, 16 queries, chunk), the
+// queries being the rows of the heads that share the kv head, so a key or
+// value is read once for 16 of them and multiplied in the MFMAs that one would
+// take. The split kernel reads it once a row and spends about 170 VALU ops a
+// wave on two positions of four heads. 64 heads on 8 of 80, 4 rows at context
+// 4096: 82 us there, 19.5 here. Bound by the latency of each wave's next
+// block: 134 MB of 32 heads' 16384 positions (8 kv heads) in 40 us, 3.4 TB/s.
+// kGroupWorkgroups fill two workgroups a CU (1024, at the registers of heads
+// of 128: 43 us against 37; 128 positions at least instead of 64: 13 against
+// 11 at context 1500, 32: 16).
+template <int E>
+__global__ __launch_bounds__(kTileWaves * kWave) void attn_group_kernel(AttnArgs a) {
+    const int kvh = blockIdx.x, cz = blockIdx.z;
+    const int last = *a.pos + a.rows - 1;
+    const int chunk = group_chunk(last + 1, a.splits, a.group_chunk_min), lo = cz * chunk;
+    if (lo > last) return;
+    const int j = blockIdx.y * kTileRows + threadIdx.x % 16;
+    tile_block<E, true>(a, kvh, kvh * a.group + j % a.group, j / a.group, last, lo,
+                        min(last, lo + chunk - 1), cz, chunk);
 }
 
 // --- prefill rows: tiles of 64 queries on bf16 MFMA -------------------------
@@ -1235,12 +1357,12 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
     const bool v_lost = __syncthreads_or((lost_v & 0xffffu) != 0) != 0;
     const bool p_lost = __ballot((lost_p & 0xffffu) != 0) != 0;
     if (__ballot(bad || (v_lost && tiny) || (p_lost && small))) {
-        tile_wave<E>(a, h, wr0, wlast, 0, wlast / 16 * 16 + 15, m, l, o);
+        tile_wave<E>(a, h / a.group, h, row, wlast, 0, wlast / 16 * 16 + 15, m, l, o);
         l = sum32(sum16(l));
-        tile_store_wave<E>(a, h, wr0, 0, m, l, o);
+        tile_store_wave<E>(a, h, wr0 + j, 0, 0, m, l, o);
         return;
     }
-    tile_store<E>(a, h, wr0, 0, m, l, [&](int u) { return 16 * u + 4 * g; },
+    tile_store<E>(a, h, wr0 + j, 0, 0, m, l, [&](int u) { return 16 * u + 4 * g; },
                   [&](int u, float f) { return o[u] * f; });
 }
 
@@ -1325,6 +1447,42 @@ void launch_split_g(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t
         case 641: launch_split<G, 64, 1, ROPE>(s, a, rows, stream); break;
         default: launch_split<G, 64, 2, ROPE>(s, a, rows, stream); break;
     }
+}
+
+// Where a few-row call runs on the grouped tile kernel, whose time follows the
+// bytes of the context, not the columns (query rows times heads of a kv head):
+// split / grouped kernel, us, heads of 128. 32 heads on 8 at context 16384: 1
+// row 38 / 39 (4 columns), 2 rows 56 / 40, 4 rows 100 / 41; 48 on 8, 1 row 72 /
+// 40; 32 on 16 at 1500 with 2 / 4 / 8 columns 13.5 / 16.4, 15.7 / 16.7, 22 /
+// 17. Heads of 64, whose keys the split kernel has less work in flight for:
+// 32 on 16 at 4096, 2 columns 16.7 / 14.2; 32 on 8, 4 columns 15.6 / 11.4. Odd
+// groups the split kernel takes a head at a time: 24 on 8 of 96, 1 row at
+// 16384 51 / 33. Contexts of 300 and less 9 - 13 either way.
+bool group_preferred(const AttnShape& s, int rows) {
+    const int group = s.n_heads / s.n_kv_heads, columns = rows * group;
+    return group >= 2 && tile_supports(s) &&
+           (columns >= (s.head_size > 64 ? 6 : 2) || heads_per_block(s) == 1);
+}
+
+// The call on the grouped tile kernel, its partials where the split kernel's
+// would be (fewer chunks, so they fit).
+void run_group(const AttnShape& s, AttnArgs a, int rows, hipStream_t stream) {
+    a.group_chunk_min = kGroupChunkMin;
+    a.splits = std::max(1, std::min(a.splits, kGroupWorkgroups / s.n_kv_heads));
+    const int columns = rows * (s.n_heads / s.n_kv_heads);
+    const dim3 grid(s.n_kv_heads, (columns + kTileRows - 1) / kTileRows, a.splits);
+    const dim3 block(kTileWaves * kWave);
+    switch (s.head_size / 16) {
+        case 1: hipLaunchKernelGGL(attn_group_kernel<1>, grid, block, 0, stream, a); break;
+        case 2: hipLaunchKernelGGL(attn_group_kernel<2>, grid, block, 0, stream, a); break;
+        case 3: hipLaunchKernelGGL(attn_group_kernel<3>, grid, block, 0, stream, a); break;
+        case 4: hipLaunchKernelGGL(attn_group_kernel<4>, grid, block, 0, stream, a); break;
+        case 5: hipLaunchKernelGGL(attn_group_kernel<5>, grid, block, 0, stream, a); break;
+        case 6: hipLaunchKernelGGL(attn_group_kernel<6>, grid, block, 0, stream, a); break;
+        case 7: hipLaunchKernelGGL(attn_group_kernel<7>, grid, block, 0, stream, a); break;
+        default: hipLaunchKernelGGL(attn_group_kernel<8>, grid, block, 0, stream, a); break;
+    }
+    if (a.splits > 1) launch_merge(s, a, rows, stream);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -1415,8 +1573,14 @@ void set_split(const AttnShape& s, int rows, float* scratch, AttnArgs& a) {
 
 void run_attention(const AttnShape& s, int rows, const int* pos, const float* q, const float* kc,
                    const float* vc, float* out, float* scratch, int kernel, hipStream_t stream) {
+    const bool automatic = kernel == kAttnAutomatic;
     kernel = resolve(kernel, rows, s);
     AttnArgs a = base_args(s, rows, pos, q, kc, vc, out);
+    if (automatic && kernel == kAttnSplit && group_preferred(s, rows)) {
+        set_split(s, rows, scratch, a);
+        run_group(s, a, rows, stream);
+        return;
+    }
     if (kernel == kAttnTile && rows_preferred(s, rows)) {
         const dim3 grid(s.n_heads, (rows + kRowsTile - 1) / kRowsTile), block(4 * kWave);
         switch (s.head_size / 16) {
