@@ -155,7 +155,8 @@ private:
 // cuda_matmul.h:66-72. The values are the C ABI's EM_KERNEL_* codes.
 enum class GpuKernel {
     automatic = EM_KERNEL_AUTOMATIC,      // fp32: skinny for m <= 8 (m <= 3 for 2^25 weights or
-                                          // more), else tiled_split (tiled if B is unaligned); int8:
+                                          // more), else a six-term bf16 split on MFMA where that
+                                          // is faster, tiled_split or tiled; int8:
                                           // skinny for 1 row and for 2-4 rows of small weights,
                                           // else exact-split bf16 MFMA
     naive = EM_KERNEL_NAIVE,              // one thread per element of C; the reference kernel

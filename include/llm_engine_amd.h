@@ -214,7 +214,8 @@ typedef struct {
 } em_attention_shape;
 
 /* Replaces enum class AttentionKernel, cuda_attention.h:15-19. */
-#define EM_ATTN_AUTOMATIC 0    /* split for up to 5 rows (12 when seq_len <= 512); more rows:
+#define EM_ATTN_AUTOMATIC 0    /* split for up to 5 rows (12 when seq_len <= 512), or 16-query
+                                  tiles over the heads of each kv head; more rows:
                                   16-row fp32 MFMA tiles, also split over the context when
                                   their grid is small (head_size a multiple of 16, at most
                                   128; large grids of heads of 64 or

@@ -1,6 +1,6 @@
 // fp32 products of many rows on bf16 matrix cores with fp32 results: what
 // GpuKernel::automatic runs for fp32 B where gemm_split_preferred says so
-// (reference: tiled / tiled_split, /root/reference/src/cuda_matmul.cu:49-125,
+// (reference: tiled / tiled_split, src/cuda_matmul.cu:49-125,
 // 350-363).
 //
 // The split. An fp32 value x is exactly hi + mid + lo, three bf16 values:
