@@ -21,8 +21,11 @@
 // that lo drops bits worth at most 2^-134. Each thread ORs what its lo terms
 // could not hold. A tile whose sums hold a non-finite value (an infinity or
 // NaN in the inputs, or an overflow), or which dropped bits and has a sum
-// below 2^-50 in magnitude (above, the drop is under a rounding of it), is
-// computed again by fp32 MFMAs straight from global memory (exact_tile).
+// below 2^-50 in magnitude or an operand of 2^37 or more, is computed again
+// by fp32 MFMAs straight from global memory (exact_tile). For the rest the
+// k < 2^21 drops of either operand add up to less than 2^21 2^-133 2^37 =
+// 2^-75, under a rounding of the sum. The operands are read again for their
+// largest value only in a tile that dropped bits.
 //
 // Speed. Six bf16 MFMAs stand for eight fp32 ones of twice the cycles each:
 // 6/16 of the fp32 MFMA time. What paces the kernel is the card's power
@@ -266,8 +269,22 @@ __global__ __launch_bounds__(kWave * WR * WC, 2) void gemm_split_kernel(GsParams
                 tiny |= x < 0x1p-50f;
             }
         }
+    // Whether this thread's share of the tile's operands holds a value of 2^37
+    // or more, by which a dropped bit could grow past that rounding.
+    auto large = [&] {
+        const int kb = cb * kChunk, ke = min(p.k, ce * kChunk);
+        const int rows = min(BM, p.m - m0), cols = min(BN, p.n - n0);
+        float top = 0.0f;
+        for (int r = w; r < rows; r += T / kWave)
+            for (int kk = kb + lane; kk < ke; kk += kWave)
+                top = fmaxf(top, fabsf(p.A[static_cast<std::size_t>(m0 + r) * p.k + kk]));
+        for (int kk = kb + w; kk < ke; kk += T / kWave)
+            for (int c = lane; c < cols; c += kWave)
+                top = fmaxf(top, fabsf(p.B[static_cast<std::size_t>(kk) * p.n + n0 + c]));
+        return top >= 0x1p37f;
+    };
     const bool dropped = __syncthreads_or((lost & 0xffffu) != 0) != 0;
-    const bool redo = __syncthreads_or(bad || (dropped && tiny)) != 0;
+    const bool redo = __syncthreads_or(bad || (dropped && (tiny || large()))) != 0;
 
     float* out = p.out + (p.direct ? 0 : static_cast<std::size_t>(place.slice) * p.m * p.n);
     const bool add = p.direct && p.accumulate;

@@ -73,6 +73,19 @@ def test_magnitudes(exponent):
           B.T, A.T)
 
 
+@pytest.mark.parametrize("exponent", [-112, -126])
+@pytest.mark.parametrize("shape", [(70, 1100, 1200), (300, 1028, 1001)], ids=str)
+def test_dropped_bits_times_large_values(shape, exponent):
+    # The bits a lo term drops below 2^-109 times values near 2^100 would show
+    # in sums far above the smallest.
+    m, k, n = shape
+    A = inputs.uniform((m, k), 1.0, 2.0, 81) * np.float32(2.0 ** exponent)
+    B = inputs.uniform((k, n), 1.0, 2.0, 82) * np.float32(2.0 ** 100)
+    check(em.matmul(dev(A), dev(B)).cpu().numpy(), A, B)
+    Bt, At = np.ascontiguousarray(B.T), np.ascontiguousarray(A.T)
+    check(em.matmul(dev(Bt), dev(At)).cpu().numpy(), Bt, At)
+
+
 def test_non_finite_values():
     m, k, n = 130, 1100, 1200
     A = inputs.uniform((m, k), 0.5, 1.0, 77)
