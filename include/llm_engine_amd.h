@@ -15,7 +15,8 @@
  * scratch buffer: concurrent calls on different streams race, as in the
  * reference (cuda_matmul.h:7-12). (The k slices of automatic's fp32 split
  * product are the exception: each stream, and each capture, has a buffer of
- * its own, 2 GiB in all; past that the product runs without slices.)
+ * its own, 2 GiB in all; past that the product runs without slices. Threads
+ * may share the stream.)
  *
  * Layout (cuda_matmul.h:94-107): A is m x k, B is k x n, C is m x n, all
  * dense row-major fp32 with no leading dimensions; int8 B carries n fp32

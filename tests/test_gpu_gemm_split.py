@@ -103,6 +103,27 @@ def test_non_finite_values():
     assert np.allclose(got[fine], want[fine], rtol=1e-5)
 
 
+def test_threads_on_one_stream():
+    # A product's slices and their sum are two launches over the stream's
+    # buffer: no other thread's product comes between them.
+    m, k, n = 200, 4096, 1024
+    A, B = dev(inputs.uniform((m, k), -1, 1, 83)), dev(inputs.uniform((k, n), -1, 1, 84))
+    As = [A * (i + 1) for i in range(4)]
+    want = [em.matmul(a, B) for a in As]
+    outs = [[torch.empty_like(want[i]) for _ in range(100)] for i in range(4)]
+    torch.cuda.synchronize()
+
+    def work(i):
+        for out in outs[i]:
+            em.matmul(As[i], B, out)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, want[i]) for i in range(4) for out in outs[i])
+
+
 def test_streams_and_threads_share_nothing():
     # Sliced products on four threads with a stream each, and a graph captured
     # without a call before it: every result equals the first stream's.
