@@ -25,7 +25,8 @@
 // by fp32 MFMAs straight from global memory (exact_tile). For the rest the
 // k < 2^21 drops of either operand add up to less than 2^21 2^-133 2^37 =
 // 2^-75, under a rounding of the sum. The operands are read again for their
-// largest value only in a tile that dropped bits.
+// largest value only in a tile that dropped bits; 2048^3 does not notice the
+// check (97.5 / 97.8 us), 300-row Llama-7B products take 775 -> 790.
 //
 // Speed. Six bf16 MFMAs stand for eight fp32 ones of twice the cycles each:
 // 6/16 of the fp32 MFMA time. What paces the kernel is the card's power
