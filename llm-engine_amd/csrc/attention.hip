@@ -1101,19 +1101,25 @@ __global__ __launch_bounds__(kTileWaves * kWave) void attn_group_kernel(AttnArgs
 //  * O^T block c: head dims 16c + 4g + r of query j.
 // The output is rescaled only when a maximum of the wave's queries moved.
 //
-// Terms below 2^-133 drop bits: scores are never that sensitive, but a value
-// (or a weight) that small may be all of an output. Where bits of V were
-// dropped and an output's sum is below 2^-50 (of P, and it is also not
-// zero), or an output or sum is not finite, the wave runs tile_wave instead.
+// Small operands drop bits: a term is a multiple of 2^-133, so a value below
+// 2^-109 is off by up to 2^-134, and exp_neg stops at e^-87, which drops bits
+// too. Where that could show, the wave runs tile_wave instead:
+//  * a query that dropped bits, whatever its keys, or one of 2^90 or more
+//    (below it, keys' dropped bits add up to less than 2^7 2^-134 2^90 =
+//    2^-37 of a score);
+//  * dropped bits of V and an output's sum below 2^-50;
+//  * dropped bits of a weight and an output's sum below 2^-99 positions times
+//    the largest value, of which n weights off by 2^-125 are up to 2^-26;
+//  * an output or sum that is not finite, or no sum at all.
 constexpr int kRowsTile = 64;
 constexpr int kRowsBlock = 32;
 
-// e^x for x <= 0 (NaN stays, 0 below 2^-126): 2^(x log2 e) with the
+// e^x for x <= 0 (NaN stays; e^floor below floor, 0 past -88): 2^(x log2 e) with the
 // rounding of the product and the rest of log2 e put back as a factor, within
 // about 2 ulp in half of expf's instructions.
-__device__ __forceinline__ float exp_neg(float x) {
+__device__ __forceinline__ float exp_neg(float x, float floor) {
     constexpr float kHi = 0x1.715476p+0f, kLo = 0x1.4ae0cp-26f, kLn2 = 0x1.62e43p-1f;
-    const float t = x < -200.0f ? -200.0f : x;
+    const float t = x < floor ? floor : x;
     const float y = t * kHi;
     const float r = fmaf(t, kLo, fmaf(t, kHi, -y));
     const float p = __builtin_amdgcn_exp2f(y);
@@ -1138,7 +1144,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
     const float* kbase = a.kc + static_cast<std::size_t>((h / a.group) * HS);
     const float* vbase = a.vc + static_cast<std::size_t>((h / a.group) * HS);
 
-    uint32_t lost_q = 0, lost_v = 0, lost_p = 0;  // lost_q is not used: see above
+    uint32_t lost_q = 0, lost_v = 0, lost_p = 0, lost_k = 0;  // lost_k is not used: see above
+    float top_q = 0.0f;
     bf16x8 q[C][3];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -1153,6 +1160,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
             v[e] = in ? x0[e] : 0.0f;
             v[4 + e] = in ? x1[e] : 0.0f;
         }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) top_q = fmaxf(top_q, fabsf(v[e]));
         uint4 t[3];
         split3x8(v, t, lost_q);
 #pragma unroll
@@ -1209,7 +1218,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
                 for (int e = 0; e < 8; ++e) v[e] = 32 * (C - 1) + 8 * uu < HS ? v[e] : 0.0f;
             }
             uint4 t[3];
-            split3x8(v, t, lost_q);
+            split3x8(v, t, lost_k);
             char* o = smem + x * 3072 + (jr * 4 + (uu ^ ((jr >> 1) & 3))) * 16;
 #pragma unroll
             for (int y = 0; y < 3; ++y) *reinterpret_cast<uint4*>(o + y * 1024) = t[y];
@@ -1277,12 +1286,22 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
         for (int e = 0; e < 8; ++e) 
             s[e] = (sh[0][e / 4][e % 4] + sh[1][e / 4][e % 4] + sl[e / 4][e % 4]) * scale;
         const int ts = start(t0);
+        // A masked position's weight is zero, so exp_neg may not stop short of
+        // that here; another weight that becomes zero then counts as one that
+        // dropped bits (found here, where it costs the other blocks nothing).
+        float floor = -87.0f;
         if (ts != t0 || t0 + kRowsBlock - 1 > pos0 + wr0) {
+            floor = -200.0f;
+            float least = INFINITY, most = m;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int t = ts + 4 * g + (e < 4 ? e : 12 + e);
-                s[e] = t >= t0 && t <= pq ? s[e] : -INFINITY;
+                const bool seen = t >= t0 && t <= pq;
+                least = fminf(least, seen ? s[e] : INFINITY);
+                s[e] = seen ? s[e] : -INFINITY;
+                most = fmaxf(most, s[e]);
             }
+            lost_p |= least - max32(max16(most)) < -87.0f;
         }
         float mb = s[0];
 #pragma unroll
@@ -1304,7 +1323,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
         float p[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            p[e] = exp_neg(s[e] - base);
+            p[e] = exp_neg(s[e] - base, floor);
             l += p[e];
         }
         uint4 t[3];
@@ -1332,6 +1351,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
     };
 
     load(0);
+    // Not after the loop, where its operands would take registers through it.
+    const bool redo_q = __ballot((lost_q & 0xffffu) != 0 || top_q >= 0x1p90f) != 0;
     for (int t0 = 0; t0 <= last; t0 += kRowsBlock) {
         __syncthreads();  // the previous block has been read
         stash();
@@ -1342,7 +1363,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
 
     // The four lane groups of query j hold parts of its sum.
     l = sum32(sum16(l));
-    bool bad = !(l < INFINITY), tiny = false, small = false;
+    bool bad = redo_q || !(l < INFINITY && l > 0.0f);
+    float low = INFINITY;
 #pragma unroll
     for (int c = 0; c < E; ++c) {
         o[c] += ol[c];
@@ -1350,13 +1372,23 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
         for (int e = 0; e < 4; ++e) {
             const float x = fabsf(o[c][e]);
             bad |= !(x < INFINITY);
-            tiny |= x < 0x1p-50f;
-            small |= x < 0x1p-50f && x > 0.0f;
+            low = fminf(low, x);
         }
     }
     const bool v_lost = __syncthreads_or((lost_v & 0xffffu) != 0) != 0;
-    const bool p_lost = __ballot((lost_p & 0xffffu) != 0) != 0;
-    if (__ballot(bad || (v_lost && tiny) || (p_lost && small))) {
+    bad |= v_lost && low < 0x1p-50f;
+    if (__ballot((lost_p & 0xffffu) != 0)) {
+        float top = 0.0f;
+#pragma unroll 1
+        for (int t = lane; t < (wlast + 1) * (HS / 4); t += kWave) {
+            const floatx4 x = *reinterpret_cast<const floatx4*>(
+                vbase + static_cast<std::size_t>(t / (HS / 4)) * a.kv_stride + t % (HS / 4) * 4);
+            top = fmaxf(fmaxf(top, fmaxf(fabsf(x[0]), fabsf(x[1]))), fmaxf(fabsf(x[2]), fabsf(x[3])));
+        }
+        for (int d = 1; d < kWave; d *= 2) top = fmaxf(top, __shfl_xor(top, d, kWave));
+        bad |= low < static_cast<float>(wlast + 1) * 0x1p-99f * top;
+    }
+    if (__ballot(bad)) {
         tile_wave<E>(a, h / a.group, h, row, wlast, 0, wlast / 16 * 16 + 15, m, l, o);
         l = sum32(sum16(l));
         tile_store_wave<E>(a, h, wr0 + j, 0, 0, m, l, o);

@@ -72,3 +72,34 @@ def test_small_and_non_finite_values():
     clean = np.ones_like(got, bool)
     clean[first // 16 * 16:, :hs] = False  # rows of the same 16 may see 0 * inf
     assert np.abs(got[clean] - want[clean]).max() <= TOL
+
+
+@pytest.mark.parametrize("exponent", [-126, -118, 118, 126])
+def test_small_queries_on_large_keys(exponent):
+    # Bits that a query's (key's) last term cannot hold below 2^-109, times
+    # keys (queries) large enough for scores of order one.
+    heads, hs, rows, pos = 256, 128, 70, 20
+    T = pos + rows
+    q, kc, vc = draw(heads, heads, hs, T, rows, 8500)
+    q, kc = q / 2 * np.float32(2.0 ** exponent), kc / 2 * np.float32(2.0 ** -exponent)
+    got = run(heads, heads, hs, T, rows, pos, q, kc, vc)
+    want = orc.attention(heads, heads, hs, rows, pos, q, kc, vc)
+    assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("score", [-70.0, -82.0, -86.5, -90.0])
+@pytest.mark.parametrize("at", [0, 40])
+def test_small_weights_on_large_values(score, at):
+    # One position far below the others' scores, its values so large that it
+    # is most of every output after it. Its score is off by a few roundings of
+    # its size (90 * 2^-24 = 5e-6 each), and so, relatively, is its weight.
+    heads, hs, rows, pos = 256, 128, 70, 20
+    T = pos + rows
+    q, kc, vc = draw(heads, heads, hs, T, rows, 8600)
+    q[:], kc[:] = 0.0, 0.0
+    q[:, 0:heads * hs:hs] = 16.0
+    kc[at, ::hs] = score * np.sqrt(np.float32(hs)) / 16.0
+    vc[at] = np.float32(2.0 ** 127) * vc[at]
+    got = run(heads, heads, hs, T, rows, pos, q, kc, vc)
+    want = orc.attention(heads, heads, hs, rows, pos, q, kc, vc)
+    assert (np.abs(got - want) <= 4e-5 * np.abs(want) + TOL).all()
