@@ -921,7 +921,9 @@ __device__ void tile_wave_plain(const AttnArgs& a, int kvh, int h, int row, int 
         }
         x = sum32(sum16(x)) * scale;
         if (t > pq) continue;
-        const float mn = fmaxf(m, x), alpha = m == mn ? 1.0f : expf(m - mn), p = expf(x - mn);
+        // A score of -inf has no weight, also where every one so far is.
+        const float mn = fmaxf(m, x), alpha = m == mn ? 1.0f : expf(m - mn);
+        const float p = x == -INFINITY ? 0.0f : expf(x - mn);
         l = l * alpha + p;
 #pragma unroll
         for (int x = 0; x < 4 * E; ++x)

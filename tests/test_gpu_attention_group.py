@@ -65,3 +65,21 @@ def test_values_a_row_does_not_see():
     assert np.isinf(got[2:, :dim]).all()
     assert np.abs(got[:2] - want[:2]).max() <= TOL
     assert np.abs(got[2:, dim:] - want[2:, dim:]).max() <= TOL
+
+
+@pytest.mark.parametrize("hs,at", [(64, 0), (64, 16), (64, 64), (128, 0), (128, 32), (128, 128)])
+def test_infinite_keys(hs, at):
+    """A key with an infinite component, at the first position of a wave's
+    part of a chunk: queries that score +inf there are NaN, those that score
+    -inf give it no weight, and both are columns of one tile."""
+    heads, kv_heads, rows, T = 16, 2, 2, 300
+    pos = T - rows
+    q, kc, vc = draw(heads, kv_heads, hs, T, rows, 8700)
+    kc[at, 0] = np.inf
+    got = run(heads, kv_heads, hs, T, rows, pos, q, kc, vc)
+    with np.errstate(invalid="ignore"):
+        want = orc.attention(heads, kv_heads, hs, rows, pos, q, kc, vc)
+    nan = np.isnan(want)
+    assert nan.any() and not nan[:, :heads // kv_heads * hs].all()
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.abs(got[~nan] - want[~nan]).max() <= TOL
