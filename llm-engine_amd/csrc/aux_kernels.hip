@@ -143,12 +143,14 @@ constexpr int kQuantRound = 16;  // rows in flight per thread
 
 // Column maxima of |B| over one slice of rows: partial[slice][4 idx + e] of
 // column column_group(idx) + e, `stride` floats to a slice. Bound by the read
-// of B (4096 x 11008: 180 MB).
+// of B (4096 x 11008: 180 MB). With W = 1, fewer than four columns, a thread
+// owns one: partial[slice][idx] of column idx.
+template <int W>
 __global__ __launch_bounds__(kThreads) void colmax_kernel(int rows, int cols, int span, int stride,
                                                           const float* B, float* partial) {
     const int idx = blockIdx.x * kThreads + threadIdx.x;
-    if (4 * idx >= stride) return;
-    const float* col = B + column_group(idx, cols);
+    if (W * idx >= stride) return;
+    const float* col = B + (W == 4 ? column_group(idx, cols) : idx);
     const int r0 = blockIdx.y * span, r1 = min(rows, r0 + span);
     // fmaxf keeps the running value when |B| is NaN, as std::max(scale, v)
     // does in quant.cpp:14; on ordered values max is exact in any order, so
@@ -157,15 +159,23 @@ __global__ __launch_bounds__(kThreads) void colmax_kernel(int rows, int cols, in
     for (int r = r0; r < r1; r += kQuantRound) {
         Floats4 x[kQuantRound];
 #pragma unroll
-        for (int u = 0; u < kQuantRound; ++u)
-            x[u] = *reinterpret_cast<const Floats4*>(col + static_cast<size_t>(min(r + u, r1 - 1)) * cols);
+        for (int u = 0; u < kQuantRound; ++u) {
+            const float* at = col + static_cast<size_t>(min(r + u, r1 - 1)) * cols;
+            if constexpr (W == 4)
+                x[u] = *reinterpret_cast<const Floats4*>(at);
+            else
+                x[u].v[0] = *at;
+        }
 #pragma unroll
         for (int u = 0; u < kQuantRound; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) mx[e] = fmaxf(mx[e], fabsf(x[u].v[e]));
+            for (int e = 0; e < W; ++e) mx[e] = fmaxf(mx[e], fabsf(x[u].v[e]));
     }
-    *reinterpret_cast<floatx4*>(partial + static_cast<size_t>(blockIdx.y) * stride + 4 * idx) =
-        floatx4{mx[0], mx[1], mx[2], mx[3]};
+    float* out = partial + static_cast<size_t>(blockIdx.y) * stride + W * idx;
+    if constexpr (W == 4)
+        *reinterpret_cast<floatx4*>(out) = floatx4{mx[0], mx[1], mx[2], mx[3]};
+    else
+        *out = mx[0];
 }
 
 // lround for the range that matters, half away from zero: x + 0.5 less one
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(kThreads) void scale_kernel(int cols, int stride, i
     }
     mx = max32(max16(mx));
     if (part != 0 || i >= stride) return;
-    const int c = column_group(i / 4, cols) + i % 4;
+    const int c = cols < 4 ? i : column_group(i / 4, cols) + i % 4;
     const float sc = mx / 127.0f;
     scale[c] = sc;
     inv[c] = sc > 0.0f ? 1.0f / sc : 0.0f;
@@ -280,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void quantize_flat_kernel(int total, int 
     }
 }
 
-// Fewer than four columns: one thread per column does it all.
+// Fewer than four columns of a few rows: one thread per column does it all.
 __global__ __launch_bounds__(kThreads) void quantize_narrow_kernel(int rows, int cols, const float* B,
                                                                    int8_t* q, float* scale) {
     const int c = threadIdx.x;
@@ -354,9 +364,13 @@ void run_fill_zero(float* p, size_t count, hipStream_t stream) {
 // address order; up to it the quantising workgroups form them. us, two
 // launches / three: 1000 x 1001 9.5 / 11.2, 300 x 11000 (19 slices) 10.4 /
 // 11.5, 11008 x 257 (256 slices) 19.5 / 15.7, 4096 x 11008 81 / 75.6 (79
-// before).
+// before). Tall matrices go the same way once a slice of a workgroup per CU is
+// deeper than kQuantDeep rows, which few of its threads then walk: 32768 x 64
+// 24 / 28, but 64000 x 4 36 / 16, 131072 x 16 59 / 18, 500000 x 4 187 / 30.
+// So do fewer than four columns past kQuantNarrow rows, against one thread a
+// column: 64 x 3 13.6 / 16.4, 300 x 1 57 / 17, 20000 x 3 3500 / 22.
 constexpr size_t kQuantSmall = size_t{1} << 21, kQuantLarge = size_t{1} << 23;
-constexpr int kQuantFewSlices = 32;
+constexpr int kQuantFewSlices = 32, kQuantDeep = 8 * kQuantRound, kQuantNarrow = 64;
 
 void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale,
                      hipStream_t stream) {
@@ -364,12 +378,13 @@ void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale
         run_fill_zero(scale, cols, stream);
         return;
     }
-    if (cols < 4) {
+    if (cols < 4 && rows <= kQuantNarrow) {
         hipLaunchKernelGGL(quantize_narrow_kernel, dim3(1), dim3(kThreads), 0, stream, rows, cols, B,
                            q, scale);
         return;
     }
-    const int stride = ceil_div(cols, 4) * 4, tiles = ceil_div(stride, 4 * kThreads);
+    const int stride = cols < 4 ? cols : ceil_div(cols, 4) * 4;
+    const int tiles = ceil_div(stride, 4 * kThreads);
     // Workgroups towards `per_cu` a CU, each with at least one round of rows.
     auto slabs = [&](int per_cu, int* span) {
         const int want = ceil_div(static_cast<long long>(per_cu) * cu_count(), tiles);
@@ -380,12 +395,13 @@ void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale
     const size_t total = static_cast<size_t>(rows) * cols;
     int span_max = 0, span = 0;
     int slices = slabs(1, &span_max);
-    const bool large = total > kQuantLarge || (total > kQuantSmall && slices > kQuantFewSlices);
+    const bool large = total > kQuantLarge || (total > kQuantSmall && slices > kQuantFewSlices) ||
+                       span_max > kQuantDeep || cols < 4;
     if (large) slices = slabs(4, &span_max);
     const int parts = slabs(2, &span);
     float* partial = scratch(kQuant, static_cast<size_t>(slices) * stride + stride);
-    hipLaunchKernelGGL(colmax_kernel, dim3(tiles, slices), dim3(kThreads), 0, stream, rows, cols,
-                       span_max, stride, B, partial);
+    hipLaunchKernelGGL(cols < 4 ? colmax_kernel<1> : colmax_kernel<4>, dim3(tiles, slices),
+                       dim3(kThreads), 0, stream, rows, cols, span_max, stride, B, partial);
     if (!large) {
         hipLaunchKernelGGL(quantize_kernel, dim3(tiles, parts), dim3(kThreads), 0, stream, rows,
                            cols, span, stride, slices, B, partial, scale, q);

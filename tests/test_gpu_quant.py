@@ -96,3 +96,30 @@ def test_ragged_shapes_with_ties_and_zero_columns(shape):
     want_q, want_s = orc.quantize_q8(B)
     assert np.array_equal(s.cpu().numpy().view(np.uint32), want_s.view(np.uint32))
     assert np.array_equal(q.cpu().numpy(), want_q)
+
+
+@pytest.mark.parametrize("shape", [(64, 3), (65, 2), (70001, 1), (60000, 2), (100003, 3), (40001, 5), (524288, 8)], ids=str)
+def test_tall_narrow_shapes(shape):
+    rows, cols = shape
+    B = inputs.uniform((rows, cols), -1.0, 1.0, 460 + cols)
+    dB = torch.from_numpy(B).cuda()
+    q, s = em.quantize_q8(dB)
+    want_q, want_s = orc.quantize_q8(B)
+    assert np.array_equal(s.cpu().numpy().view(np.uint32), want_s.view(np.uint32))
+    assert np.array_equal(q.cpu().numpy(), want_q)
+
+    # The rows are spread over the card: no slower than a few times the same
+    # values in rows of 256 (one thread a column walking them all takes
+    # hundreds of times as long).
+    def time(x):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        em.quantize_q8(x)
+        start.record()
+        for _ in range(5):
+            em.quantize_q8(x)
+        end.record()
+        torch.cuda.synchronize()
+        return start.elapsed_time(end)
+
+    wide = dB.reshape(-1)[:rows * cols // 256 * 256].reshape(-1, 256).contiguous()
+    assert time(dB) <= 20 * time(wide)
