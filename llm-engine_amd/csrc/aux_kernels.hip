@@ -365,12 +365,13 @@ void run_fill_zero(float* p, size_t count, hipStream_t stream) {
 // launches / three: 1000 x 1001 9.5 / 11.2, 300 x 11000 (19 slices) 10.4 /
 // 11.5, 11008 x 257 (256 slices) 19.5 / 15.7, 4096 x 11008 81 / 75.6 (79
 // before). Tall matrices go the same way once a slice of a workgroup per CU is
-// deeper than kQuantDeep rows, which few of its threads then walk: 32768 x 64
-// 24 / 28, but 64000 x 4 36 / 16, 131072 x 16 59 / 18, 500000 x 4 187 / 30.
-// So do fewer than four columns past kQuantNarrow rows, against one thread a
-// column: 64 x 3 13.6 / 16.4, 300 x 1 57 / 17, 20000 x 3 3500 / 22.
+// deeper than kQuantDeep rows, which few of its threads then walk (two launches
+// / three, with the calls' host work: 12000 x 32 17 / 19, 16000 x 64 18.7 /
+// 18.8, 32768 x 64 25 / 19, 131072 x 16 59 / 18, 500000 x 4 187 / 30). So do
+// fewer than four columns past kQuantNarrow rows (a thread a column / three: 64
+// x 3 13 / 16, 300 x 1 57 / 16, 20000 x 3 3500 / 22).
 constexpr size_t kQuantSmall = size_t{1} << 21, kQuantLarge = size_t{1} << 23;
-constexpr int kQuantFewSlices = 32, kQuantDeep = 8 * kQuantRound, kQuantNarrow = 64;
+constexpr int kQuantFewSlices = 32, kQuantDeep = 4 * kQuantRound, kQuantNarrow = 64;
 
 void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale,
                      hipStream_t stream) {
