@@ -14,9 +14,12 @@
  * before the GPU finishes. Calls that use split-K share one library-owned
  * scratch buffer: concurrent calls on different streams race, as in the
  * reference (cuda_matmul.h:7-12). (The k slices of automatic's fp32 split
- * product are the exception: each stream, and each capture, has a buffer of
- * its own, 2 GiB in all; past that the product runs without slices. Threads
- * may share the stream.)
+ * product are the exception: each stream has a buffer of its own, of which the
+ * 64 last used are kept, 2 GiB in all, and so has each captured graph until it
+ * and those instantiated from it are destroyed. Threads may share the stream,
+ * except with rms_weight, whose normed copy of A is in the shared scratch. A
+ * graph passed to hipGraphExecUpdate has to outlive the updated graph's
+ * launches, which use its buffer.)
  *
  * Layout (cuda_matmul.h:94-107): A is m x k, B is k x n, C is m x n, all
  * dense row-major fp32 with no leading dimensions; int8 B carries n fp32

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -314,68 +315,195 @@ namespace {
 struct StreamBuffer {
     int device;
     hipStream_t stream;
-    unsigned long long thread;   // of a hipStreamPerThread caller, 0 for a stream handle
-    unsigned long long capture;  // capture id, 0 outside one
+    unsigned long long thread;  // of a hipStreamPerThread caller, 0 for a stream handle
     float* p;
     std::size_t cap;  // floats
+    unsigned long long last;  // when it was last asked for
+};
+// A captured graph's: `graph_gone` once that graph and every one instantiated
+// or cloned from it are destroyed and their launches over.
+struct CaptureBuffer {
+    int device;
+    hipStream_t stream;
+    unsigned long long capture;
+    float* p;
+    std::size_t cap;
+    std::atomic<bool> graph_gone;
 };
 constexpr std::size_t kStreamBuffers = 64, kStreamBytes = std::size_t{2} << 30;
-std::mutex g_stream_mu;
-std::vector<StreamBuffer> g_stream_buffers;
-std::size_t g_stream_bytes = 0;  // kept in all, outgrown buffers included
+constexpr int kSpareCaptures = 16;
+
+// Never destroyed: threads and graphs may end after static objects do.
+struct Workspaces {
+    std::mutex mu;
+    std::vector<StreamBuffer> streams;
+    std::size_t bytes = 0;  // of `streams`
+    unsigned long long clock = 0;
+    std::vector<std::unique_ptr<CaptureBuffer>> captures;
+    std::vector<unsigned long long> ended;  // threads whose buffers are to be freed
+};
+Workspaces& workspaces() {
+    static Workspaces* w = new Workspaces;
+    return *w;
+}
+
+// A number of its own for each thread, never used again after it ends.
+struct ThreadNumber {
+    unsigned long long n;
+    bool used = false;  // has a buffer
+    ThreadNumber() {
+        static std::atomic<unsigned long long> threads{0};
+        n = threads.fetch_add(1) + 1;
+    }
+    ~ThreadNumber() {
+        if (!used) return;
+        Workspaces& w = workspaces();
+        std::lock_guard<std::mutex> lock(w.mu);
+        w.ended.push_back(n);
+    }
+};
+
+// Allocations under a capture, this stream's or another's, only have to be
+// allowed: they are no stream operations.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok;
+    RelaxedCapture() : ok(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+        if (!ok) (void)hipGetLastError();
+    }
+    ~RelaxedCapture() {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+float* device_floats(std::size_t floats) {
+    RelaxedCapture relaxed;
+    void* p = nullptr;
+    if (relaxed.ok && hipMalloc(&p, floats * sizeof(float)) == hipSuccess)
+        return static_cast<float*>(p);
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+// hipFree waits for the device, so for the work queued on the buffer.
+void drop(Workspaces& w, std::vector<StreamBuffer>::iterator it) {
+    RelaxedCapture relaxed;
+    if (hipFree(it->p) != hipSuccess) (void)hipGetLastError();
+    w.bytes -= it->cap * sizeof(float);
+    w.streams.erase(it);
+}
+
+// Doubling sizes, so that a caller of growing products asks for few.
+std::size_t doubled(std::size_t floats) {
+    std::size_t cap = std::size_t{1} << 20;
+    while (cap < floats) cap *= 2;
+    return cap;
+}
+
+// A stream's buffer, the least recently used ones freed where it has to be
+// allocated and would pass the bounds.
+float* stream_buffer(Workspaces& w, int device, hipStream_t stream, std::size_t floats) {
+    thread_local ThreadNumber number;
+    const unsigned long long me = stream == hipStreamPerThread ? number.n : 0;
+    auto it = std::find_if(w.streams.begin(), w.streams.end(), [&](const StreamBuffer& b) {
+        return b.device == device && b.stream == stream && b.thread == me;
+    });
+    if (it != w.streams.end()) {
+        it->last = ++w.clock;
+        if (it->cap >= floats) return it->p;
+        drop(w, it);
+    }
+    for (const unsigned long long t : w.ended)
+        for (auto b = w.streams.begin(); b != w.streams.end();) {
+            if (b->thread != t) {
+                ++b;
+                continue;
+            }
+            const auto at = b - w.streams.begin();
+            drop(w, b);
+            b = w.streams.begin() + at;
+        }
+    w.ended.clear();
+    const std::size_t cap = doubled(floats), bytes = cap * sizeof(float);
+    if (bytes > kStreamBytes) return nullptr;
+    while (w.streams.size() >= kStreamBuffers || bytes > kStreamBytes - w.bytes)
+        drop(w, std::min_element(w.streams.begin(), w.streams.end(),
+                                 [](const StreamBuffer& x, const StreamBuffer& y) {
+                                     return x.last < y.last;
+                                 }));
+    float* p = device_floats(cap);
+    if (!p) return nullptr;
+    w.streams.push_back({device, stream, me, p, cap, ++w.clock});
+    w.bytes += bytes;
+    if (me) number.used = true;
+    return p;
+}
+
+// The buffer of a capture's work on `stream`: one whose graph is gone, of a
+// capture of this stream first, then of any once kSpareCaptures are spare,
+// or new memory. The graph and those made from it keep it (a user object), so
+// graphs that replay at the same time share nothing. It is not freed: a graph
+// updated from this one (hipGraphExecUpdate) runs on it without keeping it.
+float* capture_buffer(Workspaces& w, int device, hipStream_t stream, unsigned long long capture,
+                      hipGraph_t graph, std::size_t floats) {
+    CaptureBuffer *own = nullptr, *any = nullptr;
+    int spare = 0;
+    for (const auto& b : w.captures) {
+        if (!b->graph_gone) {
+            if (b->capture == capture && b->device == device && b->stream == stream &&
+                b->cap >= floats)
+                return b->p;
+            continue;
+        }
+        ++spare;
+        if (b->device != device || b->cap < floats) continue;
+        if (!any) any = b.get();
+        if (!own && b->stream == stream) own = b.get();
+    }
+    CaptureBuffer* b = own ? own : spare >= kSpareCaptures ? any : nullptr;
+    if (!b) {
+        const std::size_t cap = doubled(floats);
+        float* p = device_floats(cap);
+        if (!p) return nullptr;
+        w.captures.emplace_back(new CaptureBuffer{device, stream, capture, p, cap, {true}});
+        b = w.captures.back().get();
+    }
+    hipUserObject_t object;
+    if (hipUserObjectCreate(&object, b,
+                            [](void* gone) { static_cast<CaptureBuffer*>(gone)->graph_gone = true; },
+                            1, hipUserObjectNoDestructorSync) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    b->stream = stream;
+    b->capture = capture;
+    b->graph_gone = false;
+    if (hipGraphRetainUserObject(graph, object, 1, hipGraphUserObjectMove) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipUserObjectRelease(object, 1);
+        return nullptr;
+    }
+    return b->p;
+}
 
 }  // namespace
 
-float* stream_workspace(hipStream_t stream, std::size_t floats) {
+StreamWorkspace::StreamWorkspace(hipStream_t stream, std::size_t floats) : lock_(workspaces().mu) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    unsigned long long id = 0;
+    unsigned long long capture = 0;
+    hipGraph_t graph = nullptr;
     int device = 0;
-    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess ||
+    if (hipStreamGetCaptureInfo_v2(stream, &status, &capture, &graph, nullptr, nullptr) !=
+            hipSuccess ||
         hipGetDevice(&device) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return;
     }
-    // A number of its own for each thread, never used again after it ends.
-    static std::atomic<unsigned long long> threads{0};
-    thread_local const unsigned long long number = threads.fetch_add(1) + 1;
-    const unsigned long long me = stream == hipStreamPerThread ? number : 0;
-    if (status == hipStreamCaptureStatusNone) id = 0;
-    std::lock_guard<std::mutex> lock(g_stream_mu);
-    auto it = std::find_if(g_stream_buffers.begin(), g_stream_buffers.end(),
-                           [&](const StreamBuffer& b) {
-                               return b.device == device && b.stream == stream &&
-                                      b.thread == me && b.capture == id;
-                           });
-    if (it != g_stream_buffers.end() && it->cap >= floats) return it->p;
-    // Doubling sizes, so the outgrown buffers add up to less than the last.
-    std::size_t cap = std::size_t{1} << 20;
-    while (cap < floats) cap *= 2;
-    const std::size_t bytes = cap * sizeof(float);
-    if (bytes > kStreamBytes - g_stream_bytes ||
-        (it == g_stream_buffers.end() && g_stream_buffers.size() >= kStreamBuffers))
-        return nullptr;
-    // An allocation is not a stream operation; under a capture it only has
-    // to be allowed.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    void* p = nullptr;
-    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
+    if (status == hipStreamCaptureStatusNone) {
+        p_ = stream_buffer(workspaces(), device, stream, floats);
+    } else if (status == hipStreamCaptureStatusActive) {
+        p_ = capture_buffer(workspaces(), device, stream, capture, graph, floats);
     }
-    const hipError_t err = hipMalloc(&p, bytes);
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (err != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    g_stream_bytes += bytes;
-    if (it == g_stream_buffers.end()) {
-        g_stream_buffers.push_back({device, stream, me, id, static_cast<float*>(p), cap});
-        return static_cast<float*>(p);
-    }
-    it->p = static_cast<float*>(p);
-    it->cap = cap;
-    return it->p;
 }
 
 std::size_t scratch_generation() { return g_generation.load(); }

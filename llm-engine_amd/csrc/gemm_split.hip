@@ -48,7 +48,7 @@
 // [term][8 k][column]. The weights are the MFMA's first operand, so a lane
 // ends up with four consecutive columns of one row.
 #include <algorithm>
-#include <mutex>
+#include <optional>
 
 #include "common.hpp"
 #include "internal.hpp"
@@ -434,13 +434,10 @@ bool gemm_split_preferred(const MatmulArgs& a) {
 void run_gemm_split(const MatmulArgs& a) {
     Plan pl = plan(a.m, a.n, a.k, true);
     float* partials = nullptr;
-    // Threads that share a stream share its buffer: each product's two launches
-    // are queued together.
-    static std::mutex pair_mu;
-    std::unique_lock<std::mutex> pair(pair_mu, std::defer_lock);
+    std::optional<StreamWorkspace> workspace;  // held until both launches are queued
     if (pl.slices > 1) {
-        pair.lock();
-        partials = stream_workspace(a.stream, static_cast<std::size_t>(pl.slices) * a.m * a.n);
+        workspace.emplace(a.stream, static_cast<std::size_t>(pl.slices) * a.m * a.n);
+        partials = workspace->p();
         if (!partials) pl = plan(a.m, a.n, a.k, false);
     }
     GsParams p{};

@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -34,14 +35,24 @@ enum ScratchSlot { kPartial = 0, kNorm = 1, kQuant = 2, kSplitA = 3, kPartialFro
                    kSlots = 5 };
 float* scratch(ScratchSlot slot, std::size_t floats);
 std::size_t scratch_generation();
-// Device memory of at least `floats` floats that only work queued on
-// `stream` uses (hipStreamPerThread: this thread's; a stream under capture:
-// that capture's), so calls on different streams do not share it, unlike
-// scratch(). Kept for the stream's next call; a buffer that grows is kept
-// too, since a captured graph may hold it. Null, nothing allocated, past 64
-// streams or 2 GiB in all, or if the memory cannot be had: the caller then
-// does without.
-float* stream_workspace(hipStream_t stream, std::size_t floats);
+// Device memory of at least `floats` floats that only work queued on `stream`
+// uses (hipStreamPerThread: this thread's; a stream under capture: that
+// capture's), so calls on different streams do not share it, unlike
+// scratch(). The caller queues what uses it before this object ends: until
+// then no other thread gets or frees a buffer, so that threads may share a
+// stream. A stream's buffer stays for its next call while it is among the 64
+// last used, 2 GiB in all, or until a thread with its own default stream
+// ends; a capture's as long as its graph, then it serves another capture.
+// p() is null where the memory cannot be had: the caller then does without.
+class StreamWorkspace {
+public:
+    StreamWorkspace(hipStream_t stream, std::size_t floats);
+    float* p() const { return p_; }
+
+private:
+    std::lock_guard<std::mutex> lock_;
+    float* p_ = nullptr;
+};
 // Library-owned arrival counters for one-launch split-K products: `count`
 // 32-bit words, zero. Grow-only like scratch() (growth bumps
 // scratch_generation()); zeroed when allocated, and every call leaves the

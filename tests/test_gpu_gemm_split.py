@@ -7,6 +7,7 @@ six terms a chunk in two accumulators of which only hi * hi is full size; the
 slices' sum and the prior C add one each, the left-out terms 2^-26. So
 (k / 16 + 24) * 2^-24 * sum |a||b| holds with room (the sums are rarely at
 their largest throughout)."""
+import ctypes
 import threading
 
 import numpy as np
@@ -156,3 +157,73 @@ def test_streams_and_threads_share_nothing():
         torch.cuda.synchronize()
         assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
         em.matmul(As[2], B)
+
+
+def test_captures_threads_and_streams_give_their_slices_back():
+    # Graphs captured and destroyed, threads that ran on their own default
+    # stream and ended, and more streams than keep a buffer: none changes what
+    # any product gives, and the memory stays bounded.
+    m, k, n = 200, 4096, 1024
+    A, B = dev(inputs.uniform((m, k), -1, 1, 85)), dev(inputs.uniform((k, n), -1, 1, 86))
+    A2 = A * 2
+    want, want2 = em.matmul(A, B), em.matmul(A2, B)
+    out, out2 = torch.empty_like(want), torch.empty_like(want)
+    torch.cuda.synchronize()
+
+    def capture(a, o):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            em.matmul(a, B, o)
+        return g
+
+    def replay(g, o, w):
+        o.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, w)
+
+    def captures(count):
+        kept = capture(A2, out2)
+        for _ in range(count):
+            replay(capture(A, out), out, want)
+        replay(kept, out2, want2)
+
+    def product(stream, mine):
+        em.matmul_f32_raw(m, n, k, A.data_ptr(), B.data_ptr(), mine.data_ptr(), "automatic",
+                          False, None, stream)
+        em.synchronize()
+
+    def threads(count):
+        for _ in range(count):
+            mine = torch.zeros_like(want)
+            torch.cuda.synchronize()
+            t = threading.Thread(target=product, args=(em.STREAM_PER_THREAD, mine))
+            t.start()
+            t.join()
+            assert torch.equal(mine, want)
+
+    def streams(count):
+        cudart, handles = torch.cuda.cudart(), []
+        mine = torch.zeros_like(want)
+        for _ in range(count):
+            h = ctypes.c_void_p()
+            assert int(cudart.cudaStreamCreate(ctypes.addressof(h))) == 0
+            handles.append(h)
+            mine.zero_()
+            torch.cuda.synchronize()
+            product(h.value, mine)
+            assert torch.equal(mine, want)
+        for h in handles:
+            assert int(cudart.cudaStreamDestroy(h.value)) == 0
+
+    captures(20), threads(4)
+    free = torch.cuda.mem_get_info()[0]
+    captures(70), threads(70)
+    # A buffer is 4 MiB, so 140 kept ones would be 560; the rest is a graph's
+    # end being noticed late, and the runtime's own.
+    assert free - torch.cuda.mem_get_info()[0] < 140 << 20
+    streams(70)
+    captures(4), threads(4)
+    replay(capture(A2, out2), out2, want2)
+    assert torch.equal(em.matmul(A, B), want)
+    assert free - torch.cuda.mem_get_info()[0] < 2 << 30
