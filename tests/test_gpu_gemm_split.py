@@ -4,7 +4,7 @@ operands into bf16 terms (csrc/gemm_split.hip), against 64-bit products.
 Bound per element: every MFMA adds its 32 products to an fp32 accumulator
 with at most two roundings of 2^-24 each at the size of the sums so far, and
 six terms a chunk in two accumulators of which only hi * hi is full size; the
-slices' sum and the prior C add one each, the left-out terms 2^-26. So
+slices' sum and the prior C add one each, the left-out terms at most one. So
 (k / 16 + 24) * 2^-24 * sum |a||b| holds with room (the sums are rarely at
 their largest throughout)."""
 import ctypes
@@ -157,6 +157,16 @@ def test_streams_and_threads_share_nothing():
         torch.cuda.synchronize()
         assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
         em.matmul(As[2], B)
+
+
+def test_left_out_terms_of_one_sign():
+    # 0x1.00ff8p+0 = 1 + 2^-8 - 2^-17: mid and lo at their largest, and every
+    # left-out sum 2^-24 of its product and of one sign.
+    for m, k, n in [(9, 32, 40000), (300, 1028, 1001), (200, 4096, 1024)]:
+        A = np.full((m, k), float.fromhex("0x1.00ff8p+0"), np.float32)
+        B = np.full((k, n), float.fromhex("0x1.00ff8p+0"), np.float32)
+        check(em.matmul(dev(A), dev(B)).cpu().numpy(), A, B)
+        check(em.matmul(dev(A), dev(-B)).cpu().numpy(), A, -B)
 
 
 def test_captures_threads_and_streams_give_their_slices_back():
