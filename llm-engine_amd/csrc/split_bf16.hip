@@ -1040,6 +1040,12 @@ bool split_bf16_swiglu_supported(const MatmulArgs& a, int hidden) {
            split_bf16_supports(a) && reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
 }
 
+// Planned as the product alone: where slices win there, the SwiGLU's own kernel
+// does not cost what they gain. Forward passes with slices and swiglu_kernel /
+// with the pair in one slice, us: four layers of 4096 x 22016 at 33 / 40 / 48
+// rows 578 / 615, 590 / 621, 605 / 632; two of 5120 x 27648 370 / 406, 402 /
+// 433, 406 / 436; four of 2048 x 11264 at 17 .. 80 rows and six of 1024 x 5632
+// the same within 1 %.
 bool run_split_bf16_swiglu(const MatmulArgs& a, int hidden) {
     if (!split_bf16_swiglu_supported(a, hidden)) return false;
     bool fused = false;
