@@ -17,6 +17,7 @@ import subprocess
 import pytest
 
 from tests import e2e_model
+from tests.test_cpp_drop_in import need
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 REF = os.path.join(ROOT, "oracle", "_ref")
@@ -25,8 +26,7 @@ GPU_BIN = os.path.join(REF, "stories_gpu")
 
 
 def run(binary, ckpt, prompt, wtype, n_decode):
-    if not os.path.exists(binary):
-        pytest.fail(f"{binary} is not built (make -C oracle e2e)")
+    need(binary)
     r = subprocess.run([binary, ckpt, prompt, wtype, str(n_decode)], capture_output=True,
                        text=True, timeout=900)
     assert r.returncode == 0, r.stdout + r.stderr
