@@ -376,17 +376,19 @@ struct Plan {
 // the partials' traffic at 6 TB/s and a 2 us launch. Slices are at least
 // four chunks deep. For the 300-row Llama-7B products it picks the fastest
 // shape and slices of those measured.
-// Past two workgroups a CU, more slices only add traffic.
+// Past two workgroups a CU, more slices only add traffic. A few narrow tiles
+// of a deep k take up to 64 (at most 16: 12 x 13000 x 256 25 us against 11.6
+// now and 12.3 for tiled_split), every fourth past 16 to keep the search short.
 Plan plan(int m, int n, int k, bool slices_ok) {
     const unsigned chunks = ceil_div(k, kChunk), cus = cu_count();
     Plan best{nullptr, 1, static_cast<int>(chunks), 0.0};
     for (const Shape& sh : kShapes) {
         const unsigned tiles = static_cast<unsigned>(ceil_div(m, sh.bm)) * ceil_div(n, sh.bn);
         const unsigned most =
-            slices_ok ? std::max(1u, std::min({16u, chunks / 4, 2 * cus / tiles + 1})) : 1u;
-        for (unsigned slices = 1; slices <= most; ++slices) {
-            const unsigned span = (chunks + slices - 1) / slices;
-            if (span * (slices - 1) >= chunks) continue;  // fewer slices cover k
+            slices_ok ? std::max(1u, std::min({64u, chunks / 4, 2 * cus / tiles + 1})) : 1u;
+        for (unsigned want = 1; want <= most; want += want < 16 ? 1 : 4) {
+            const unsigned span = (chunks + want - 1) / want;
+            const unsigned slices = (chunks + span - 1) / span;
             const unsigned groups = tiles * slices;
             double rounds_us;
             unsigned rounds;
@@ -422,13 +424,27 @@ bool gemm_split_supports(const MatmulArgs& a) {
 //    4096^2 at m = 32 / 300 / 1024 25 / 22, 135 / 70, 263 / 177; 4096 x
 //    11008 at m = 48 / 300 / 2048 80 / 55, 266 / 185, 1337 / 935; 3000 x
 //    3001 at m = 17 / 700 42 / 15, 222 / 104.
+//  - Without float4 stores past about 640 k^2 outputs the stores cost more than
+//    the split gains: 956 x 64 x 3895 14.6 / 17.0, 1916 x 48 x 13122 47 / 92.
+//    By n alone: an output off 16 bytes gives the same bits as one that is
+//    not (so does 1100 x 32 x 40000, 49 / 67, which stays here).
+//  - A shallow product whose 64 x 64 tiles are one round of the streamlined
+//    tiled kernel (a quarter more up to k = 640): 298 x 448 x 3040 11.7 / 17.1,
+//    440 x 512 x 2368 21.1 / 24.3, 302 x 896 x 2688 24.2 / 27.0, and a whole
+//    round 295 x 1088 x 3264 27.1 / 31.2; with fewer than 5/8 of one, or
+//    deeper, the split wins (k = 2048 and a round 0.85).
 //  - At few rows tiled_split streams the weights with less work per byte:
 //    m = 16 2048 x 4096 14.3 / 13.4 but 4096^2 20.1 / 22.0 and 4096 x 11008
 //    35 / 41; m = 24 4096 x 11008 41.8 / 41.0, m = 17 5120 x 13824 53 / 57.
 bool gemm_split_preferred(const MatmulArgs& a) {
     const long long w = static_cast<long long>(a.n) * a.k;
     if (a.m <= 8 || !gemm_split_supports(a)) return false;
+    if (a.n % 4 && static_cast<long long>(a.m) * a.n > 640LL * a.k * a.k) return false;
     if (w <= (1LL << 20)) return !tiled_preferred(a);
+    const int tiles = ceil_div(a.m, 64) * ceil_div(a.n, 64), cus = cu_count();
+    if (a.k <= (16 * tiles > 15 * cus ? 1300 : 900) && 8 * tiles > 5 * cus && tiles <= cus + (a.k <= 640 ? cus / 4 : 0) &&
+        tiled_preferred(a))
+        return false;
     return w <= (1LL << 23) || a.m > 32 || (a.m > 16 && w < (1LL << 26)) ||
            !tiled_split_supports<float>(a);
 }

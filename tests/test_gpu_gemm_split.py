@@ -61,6 +61,21 @@ def test_tile_edges(shape):
     assert torch.equal(off, first)
 
 
+# A few narrow tiles of a deep k: tens of k slices, the last ones short.
+@pytest.mark.parametrize("shape", [(9, 13000, 200), (12, 10912, 128), (33, 12004, 97), (64, 9000, 520)],
+                         ids=str)
+def test_many_slices(shape):
+    m, k, n = shape
+    A, B = inputs.uniform((m, k), -1.0, 1.0, 87), inputs.uniform((k, n), -1.0, 1.0, 88)
+    C0 = inputs.uniform((m, n), -4.0, 4.0, 89)
+    first = em.matmul(dev(A), dev(B))
+    check(first.cpu().numpy(), A, B)
+    assert torch.equal(first, em.matmul(dev(A), dev(B)))
+    C = dev(C0.copy())
+    em.matmul(dev(A), dev(B), C, accumulate=True)
+    check(C.cpu().numpy(), A, B, C0)
+
+
 @pytest.mark.parametrize("exponent", [-100, -115, -126, 40])
 def test_magnitudes(exponent):
     # Below 2^-109 a lo term drops bits; the product must not. With B scaled
