@@ -327,7 +327,9 @@ __global__ __launch_bounds__(kThreads, PIPE && G <= 4 ? 4 : 1) void attn_split_k
     const int hs = a.head_size, hs4 = hs / 4;
     const int hg = blockIdx.x, i = blockIdx.y, s = blockIdx.z;
     const int n_ctx = *a.pos + i + 1;
-    const int chunk = n_ctx <= a.whole ? n_ctx : split_chunk(n_ctx, a.splits, a.min_chunk);
+    // Only ROPE calls set `whole`. (Testing it in the others too cost heads of
+    // 256 10 % by the registers that the compiler then gave their loads.)
+    const int chunk = ROPE && n_ctx <= a.whole ? n_ctx : split_chunk(n_ctx, a.splits, a.min_chunk);
     const int t0 = s * chunk;
     if (t0 >= n_ctx) return;  // uniform across the workgroup
     const int len = min(chunk, n_ctx - t0);
