@@ -1444,10 +1444,13 @@ void launch_merge(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t s
 // 135 / 121, of 32 on 8 kv heads of 128 82 / 77; one row of 32 heads of 64 at
 // 9000 37.7 / 33.5. Not for one row of two or four heads of 128 a workgroup,
 // whose four-deep grid already overlaps (8 kv heads at 9000 / 16384 28.2 /
-// 29.6, 37.8 / 40.9), nor past 128 dims, where it spills.
+// 29.6, 37.8 / 40.9), nor past 128 dims, where it spills, nor for a prompt's
+// rows, which fill the card with workgroups (489 rows of 48 heads of 40 at
+// context 5802 4397 / 6004).
 template <int G, int LPP>
 constexpr bool split_pipes(int rows) {
-    return LPP <= 32 && (rows > 1 || G == 1 || G == 8 || LPP <= 16);
+    return LPP <= 32 && rows <= static_cast<int>(kSplitMaxRows) &&
+           (rows > 1 || G == 1 || G == 8 || LPP <= 16);
 }
 
 // Rows of fewer than a.merge_from chunks are left for the caller to merge;
@@ -1463,7 +1466,7 @@ void launch_split(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t s
             hipLaunchKernelGGL((attn_split_kernel<G, LPP, F, ROPE, true>), grid, dim3(kThreads), lds,
                                stream, a);
     }
-    if constexpr (!split_pipes<G, LPP>(1)) {
+    if constexpr (!ROPE || !split_pipes<G, LPP>(1)) {
         if (!piped)
             hipLaunchKernelGGL((attn_split_kernel<G, LPP, F, ROPE>), grid, dim3(kThreads), lds, stream,
                                a);
