@@ -1409,11 +1409,15 @@ __global__ __launch_bounds__(4 * kWave, 2) void attn_rows_kernel(AttnArgs a) {
 // 301; 1024 rows 137 / 86 and at 4096 706 / 371; 256 rows at 1024 56 / 80.
 // Heads of 64 (half the MFMAs beside the same softmax): 1024 rows at 1024 /
 // 4096 54 / 49, 329 / 224, but 512 rows 47 / 54; of 48, 1024 rows of 6 heads
-// 31 / 50.
+// 31 / 50. Heads of 112 pad their last 32 dims: 16 and 24 of them, 1057 and
+// 775 rows at their own length 68 / 82, 54 / 60; from 1.5 workgroups a CU 0.9
+// of the tile kernel's time and less.
 bool rows_preferred(const AttnShape& s, int rows) {
     const long long tiles = static_cast<long long>(s.n_heads) * ((rows + kRowsTile - 1) / kRowsTile);
-    return rows >= kRowsBlock &&
-           (s.head_size >= 112 ? tiles >= cu_count() : s.head_size >= 64 && tiles >= 2 * cu_count());
+    const long long least = s.head_size >= 128   ? cu_count()
+                            : s.head_size >= 112 ? cu_count() * 3 / 2
+                                                 : 2 * cu_count();
+    return rows >= kRowsBlock && s.head_size >= 64 && tiles >= least;
 }
 
 void launch_tile(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t stream) {

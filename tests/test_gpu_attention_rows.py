@@ -38,7 +38,7 @@ def draw(heads, kv_heads, hs, T, rows, seed):
 # Head sizes that fill their 32-dim chunks and 80, 112 that do not; rows at
 # the least the kernel takes, around a 16-row wave, a tile and two; contexts
 # around 32-position blocks, the end of the cache exactly at one and past it.
-CASES = [(512, 512, 64), (512, 64, 80), (640, 640, 96), (256, 32, 112), (256, 256, 128)]
+CASES = [(512, 512, 64), (512, 64, 80), (640, 640, 96), (256, 32, 112), (384, 32, 112), (256, 256, 128)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
