@@ -1500,10 +1500,14 @@ void launch_split_g(const AttnShape& s, const AttnArgs& a, int rows, hipStream_t
 // 17. Heads of 64, whose keys the split kernel has less work in flight for:
 // 32 on 16 at 4096, 2 columns 16.7 / 14.2; 32 on 8, 4 columns 15.6 / 11.4. Odd
 // groups the split kernel takes a head at a time: 24 on 8 of 96, 1 row at
-// 16384 51 / 33. Contexts of 300 and less 9 - 13 either way.
+// 16384 51 / 33. Short contexts, 2 to 4 rows: heads of 64 at 50 5.3 / 4.9, of 96
+// and 112 at 50 5.2 / 6.3, at 300 the same, of 128 at 50 5.2 / 7.2, at 250 8.6 /
+// 9.8, at 700 the same. The context is not known here, so a cache that holds
+// no longer ones leaves the larger heads to the split kernel.
 bool group_preferred(const AttnShape& s, int rows) {
     const int group = s.n_heads / s.n_kv_heads, columns = rows * group;
-    return group >= 2 && tile_supports(s) &&
+    const int cache = s.head_size <= 80 ? 0 : s.head_size <= 112 ? 256 : 1024;
+    return group >= 2 && tile_supports(s) && s.seq_len > cache &&
            (columns >= (s.head_size > 64 ? 6 : 2) || heads_per_block(s) == 1);
 }
 

@@ -38,7 +38,7 @@ def draw(heads, kv_heads, hs, T, rows, seed):
 
 # heads, kv heads, head size, rows, cache: columns 2, 3, 6, 15, 16, 17, 35, 96.
 CASES = [(2, 1, 16, 1, 900), (6, 2, 96, 1, 900), (12, 4, 112, 2, 900), (15, 3, 48, 3, 900),
-         (32, 8, 128, 4, 900), (17, 1, 80, 1, 900), (14, 2, 64, 5, 900), (16, 2, 32, 12, 500)]
+         (32, 8, 128, 4, 900), (32, 8, 128, 4, 1100), (17, 1, 80, 1, 900), (14, 2, 64, 5, 900), (16, 2, 32, 12, 500)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
@@ -72,8 +72,7 @@ def test_infinite_keys(hs, at):
     """A key with an infinite component, at the first position of a wave's
     part of a chunk: queries that score +inf there are NaN, those that score
     -inf give it no weight, and both are columns of one tile."""
-    heads, kv_heads, rows, T = 16, 2, 2, 300
-    pos = T - rows
+    heads, kv_heads, rows, T, pos = 16, 2, 2, 1100, 298
     q, kc, vc = draw(heads, kv_heads, hs, T, rows, 8700)
     kc[at, 0] = np.inf
     got = run(heads, kv_heads, hs, T, rows, pos, q, kc, vc)
