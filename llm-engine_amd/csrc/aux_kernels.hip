@@ -368,10 +368,11 @@ void run_fill_zero(float* p, size_t count, hipStream_t stream) {
 // deeper than kQuantDeep rows, which few of its threads then walk (two launches
 // / three, with the calls' host work: 12000 x 32 17 / 19, 16000 x 64 18.7 /
 // 18.8, 32768 x 64 25 / 19, 131072 x 16 59 / 18, 500000 x 4 187 / 30). So do
-// fewer than four columns past kQuantNarrow rows (a thread a column / three: 64
-// x 3 13 / 16, 300 x 1 57 / 16, 20000 x 3 3500 / 22).
+// fewer than four columns past kQuantNarrow rows (a thread a column / three;
+// on the card alone 16 x 3 3.2 / 5.2, 64 x 3 8 / 5.4; 300 x 1 57 / 16, 20000 x 3
+// 3500 / 22).
 constexpr size_t kQuantSmall = size_t{1} << 21, kQuantLarge = size_t{1} << 23;
-constexpr int kQuantFewSlices = 32, kQuantDeep = 4 * kQuantRound, kQuantNarrow = 64;
+constexpr int kQuantFewSlices = 32, kQuantDeep = 4 * kQuantRound, kQuantNarrow = 32;
 
 void run_quantize_q8(int rows, int cols, const float* B, int8_t* q, float* scale,
                      hipStream_t stream) {

@@ -98,7 +98,7 @@ def test_ragged_shapes_with_ties_and_zero_columns(shape):
     assert np.array_equal(q.cpu().numpy(), want_q)
 
 
-@pytest.mark.parametrize("shape", [(64, 3), (65, 2), (70001, 1), (60000, 2), (100003, 3), (40001, 5), (524288, 8)], ids=str)
+@pytest.mark.parametrize("shape", [(32, 3), (33, 2), (70001, 1), (60000, 2), (100003, 3), (40001, 5), (524288, 8)], ids=str)
 def test_tall_narrow_shapes(shape):
     rows, cols = shape
     B = inputs.uniform((rows, cols), -1.0, 1.0, 460 + cols)
