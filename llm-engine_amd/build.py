@@ -10,7 +10,7 @@ hipcc line links the shared library next to this file. Flags:
   --offload-arch=gfx950                 CDNA4 only
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                         no v_pk_*_f32 (packed fp32 ops have given
-                                        wrong results on these boxes)
+                                        wrong results on gfx950)
   -fhip-fp32-correctly-rounded-divide-sqrt
                                         IEEE division: quantize_q8's scale and
                                         reciprocal must round as the CPU's do

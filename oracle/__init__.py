@@ -11,7 +11,7 @@ Two libraries sit behind it:
 * ``_ref/libref_v{3,4}.so`` -- the reference's own ``matmul.cpp``,
   ``quant.cpp``, ``thread_pool.cpp`` and ``ops.cpp`` compiled from source by
   ``oracle/Makefile`` (amdclang++ -O3), behind ``ref_shim.cpp``. Present in
-  the build container and shipped prebuilt to the GPU box; ``ref()`` returns
+  the reference lies and shipped prebuilt elsewhere; ``ref()`` returns
   None where it is missing.
 """
 from __future__ import annotations
