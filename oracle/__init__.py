@@ -10,7 +10,7 @@ Two libraries sit behind it:
   matmul.cpp:205-217, ops.cpp:8-26 of the reference).
 * ``_ref/libref_v{3,4}.so`` -- the reference's own ``matmul.cpp``,
   ``quant.cpp``, ``thread_pool.cpp`` and ``ops.cpp`` compiled from source by
-  ``oracle/Makefile`` (amdclang++ -O3), behind ``ref_shim.cpp``. Present in
+  ``oracle/Makefile`` (amdclang++ -O3), behind ``ref_shim.cpp``. Present where
   the reference lies and shipped prebuilt elsewhere; ``ref()`` returns
   None where it is missing.
 """
